@@ -832,7 +832,7 @@ def main() -> int:
                     help="run only the bee-scale renderFrame workload (profiler runs of k_render_tasks)")
     ap.add_argument("--no-split", action="store_true", help="disable split launches (chunks of a unit on several waves)")
     ap.add_argument("--trace-mode", type=int, default=2, choices=(0, 1, 2),
-                    help="renderFrame traversal: 0 per-ray, 1 wave packets, 2 wave packets with scalar node loads "
+                    help="renderFrame traversal: 0 per-ray, 1 wave packets, 2 wave packets on the 64-wide tree "
                          "(default)")
     ap.add_argument("--copy-probe", type=float, default=0.0,
                     help="also run a plain copy kernel of this many MiB (profiler bandwidth reference)")

@@ -27,6 +27,7 @@ SOURCES = [
     "scene_loader.cpp",
     "scan.hip",
     "lbvh.hip",
+    "wide_bvh.hip",
     "render.hip",
     "projection.hip",
     "batch.cpp",

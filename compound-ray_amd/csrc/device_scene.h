@@ -9,6 +9,7 @@
 
 #include "bvh_format.h"
 #include "eyecore.h"
+#include "wide_bvh.h"
 
 namespace eye {
 
@@ -24,6 +25,16 @@ struct DeviceScene {
   float4* cols = nullptr;
   uint32_t* sorted_ids = nullptr;  // sorted position -> original triangle id
   uint32_t* codes = nullptr;       // sorted Morton codes
+  // The packets' 64-wide tree (wide_bvh.h), root wide_root; its triangles in
+  // its own order, three float4 each, a row per axis: (v0.x, v1.x, v2.x,
+  // original id), (v0.y, v1.y, v2.y, canonical position: the index into
+  // cols), (v0.z, v1.z, v2.z, 0).
+  WideNode64* wide_nodes = nullptr;
+  float4* wide_tris = nullptr;
+  int wide_count = 0;
+  int wide_root = 0;
+  int wide_stack = 0;              // deferred children any packet can hold
+  float wide_radius = 0.0f;        // the boxes' padding covers origins out to 4 of it
   int tri_count = 0;
   int stack_bound = 0;             // deepest traversal stack any ray can need
   int levels = 0;

@@ -1650,7 +1650,7 @@ int setSceneLeafSize(int leafSize) {
 }
 
 void setTraversalMode(int mode) {
-  set_trace_mode(mode == 0 ? kTracePerRay : mode == 2 ? kTracePacketScalar : kTracePacket);
+  set_trace_mode(mode == 0 ? kTracePerRay : mode == 2 ? kTracePacketWide : kTracePacket);
 }
 
 void setSampleRecording(bool enabled) { st().record_samples = enabled; }

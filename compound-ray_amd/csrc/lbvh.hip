@@ -10,7 +10,9 @@
 #include <vector>
 
 #include "device_scene.h"
+#include "radix.h"
 #include "scan.h"
+#include "wide_bvh.h"
 
 namespace eye {
 namespace {
@@ -23,12 +25,6 @@ namespace {
       return false;                                                                \
     }                                                                              \
   } while (0)
-
-constexpr int kSortThreads = 256;
-constexpr int kSortItems = 8;
-constexpr int kSortTile = kSortThreads * kSortItems;
-constexpr int kRadix = 256;
-constexpr int kWaves = kSortThreads / 64;
 
 // Deterministic min/max (ties return the second operand), identical on the CPU.
 __device__ __forceinline__ float dmin(float a, float b) { return a < b ? a : b; }
@@ -136,81 +132,6 @@ __global__ void k_morton(const float* __restrict__ cen, int n, const uint32_t* _
   }
   codes[i] = morton30(cen[3 * (size_t)i], cen[3 * (size_t)i + 1], cen[3 * (size_t)i + 2], lo, hi);
   ids[i] = (uint32_t)i;
-}
-
-// Per-tile digit histogram, written digit-major: hist[digit * tiles + tile].
-__global__ __launch_bounds__(kSortThreads) void k_sort_hist(const uint32_t* __restrict__ keys, int n,
-                                                            int shift, uint32_t* __restrict__ hist,
-                                                            int tiles) {
-  __shared__ uint32_t h[kRadix];
-  h[threadIdx.x] = 0;
-  __syncthreads();
-  const size_t base = (size_t)blockIdx.x * kSortTile;
-  for (int j = 0; j < kSortItems; ++j) {
-    const size_t idx = base + (size_t)j * kSortThreads + threadIdx.x;
-    if (idx < (size_t)n) atomicAdd(&h[(keys[idx] >> shift) & (kRadix - 1)], 1u);
-  }
-  __syncthreads();
-  hist[(size_t)threadIdx.x * tiles + blockIdx.x] = h[threadIdx.x];
-}
-
-// Stable scatter.  Items are taken in the order (item j, wave, lane); ranks
-// among equal digits inside a wave come from ballot matching, across waves
-// and items from LDS running counters, across tiles from the scanned
-// histogram.
-__global__ __launch_bounds__(kSortThreads) void k_sort_scatter(
-    const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin, uint32_t* __restrict__ kout,
-    uint32_t* __restrict__ vout, int n, int shift, const uint32_t* __restrict__ offs, int tiles) {
-  __shared__ uint32_t wave_cnt[kWaves][kRadix];
-  __shared__ uint32_t wave_off[kWaves][kRadix];
-  __shared__ uint32_t run_base[kRadix];
-  __shared__ uint32_t g_off[kRadix];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int w = tid >> 6;
-  run_base[tid] = 0;
-  g_off[tid] = offs[(size_t)tid * tiles + blockIdx.x];
-  const uint64_t lt_mask = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
-  const size_t base = (size_t)blockIdx.x * kSortTile;
-  for (int j = 0; j < kSortItems; ++j) {
-    const size_t idx = base + (size_t)j * kSortThreads + tid;
-    const bool valid = idx < (size_t)n;
-    const uint32_t key = valid ? kin[idx] : 0u;
-    const uint32_t val = valid ? vin[idx] : 0u;
-    const uint32_t d = (key >> shift) & (kRadix - 1);
-    for (int k = 0; k < kWaves; ++k) wave_cnt[k][tid] = 0;
-    __syncthreads();
-    uint64_t peers = __ballot(valid);
-    for (int b = 0; b < 8; ++b) {
-      const bool bit = (d >> b) & 1u;
-      const uint64_t m = __ballot(bit);
-      peers &= bit ? m : ~m;
-    }
-    uint32_t rank = 0;
-    if (valid) {
-      rank = (uint32_t)__popcll(peers & lt_mask);
-      const int leader = 63 - __clzll((long long)peers);
-      if (leader == lane) wave_cnt[w][d] = (uint32_t)__popcll(peers);
-    }
-    __syncthreads();
-    {
-      uint32_t run = run_base[tid];
-      for (int k = 0; k < kWaves; ++k) {
-        const uint32_t c = wave_cnt[k][tid];
-        wave_off[k][tid] = run;
-        run += c;
-      }
-      run_base[tid] = run;
-    }
-    __syncthreads();
-    if (valid) {
-      const uint32_t pos = g_off[d] + wave_off[w][d] + rank;
-      if (pos < (uint32_t)n) {  // always true for a consistent histogram; never write out of bounds
-        kout[pos] = key;
-        vout[pos] = val;
-      }
-    }
-  }
 }
 
 __global__ void k_karras(const uint32_t* __restrict__ codes, int n, int32_t* __restrict__ left,
@@ -442,6 +363,7 @@ void free_device_scene(DeviceScene* s) {
   if (s->cols) (void)hipFree(s->cols);
   if (s->sorted_ids) (void)hipFree(s->sorted_ids);
   if (s->codes) (void)hipFree(s->codes);
+  free_wide_tree(s);
   *s = DeviceScene();
 }
 
@@ -537,9 +459,9 @@ bool build_device_scene(const float* d_pos, const float* d_col, const uint32_t* 
       uint32_t *kin = codes_a, *kout = codes_b, *vin = ids_a, *vout = ids_b;
       bool sort_ok = true;
       for (int shift = 0; shift < 30; shift += 8) {
-        hipLaunchKernelGGL(k_sort_hist, dim3(tiles), dim3(kSortThreads), 0, stream, kin, n, shift, hist, tiles);
+        hipLaunchKernelGGL(k_sort_hist<uint32_t>, dim3(tiles), dim3(kSortThreads), 0, stream, kin, n, shift, hist, tiles);
         if (!scan_exclusive_u32(&scan, hist, (size_t)kRadix * tiles, stream, err)) { sort_ok = false; break; }
-        hipLaunchKernelGGL(k_sort_scatter, dim3(tiles), dim3(kSortThreads), 0, stream, kin, vin, kout, vout, n,
+        hipLaunchKernelGGL(k_sort_scatter<uint32_t>, dim3(tiles), dim3(kSortThreads), 0, stream, kin, vin, kout, vout, n,
                            shift, hist, tiles);
         uint32_t* t = kin; kin = kout; kout = t;
         t = vin; vin = vout; vout = t;
@@ -652,6 +574,11 @@ bool build_device_scene(const float* d_pos, const float* d_col, const uint32_t* 
   out->node_count = node_total;
   out->stack_bound = host_sb;
   out->levels = level_count;
+  // the tree that eye rays walk, over the same triangles
+  if (!build_wide_tree(out, stream, err)) {
+    free_device_scene(out);
+    return false;
+  }
   out->build_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   return true;
 }

@@ -104,10 +104,10 @@ struct UnitLaunch {
   unsigned long long* packet_counts = nullptr;
 };
 
-// Traversal inside the unit renderer: the wave walks the BVH as one packet
-// (a wave-uniform node, node records read with vector loads or through the
-// scalar unit), or every lane walks its own ray with an LDS stack per lane.
-enum UnitTraversal : int { kUnitPacket = 0, kUnitPacketScalar = 1, kUnitPerRay = 2 };
+// Traversal inside the unit renderer: the wave walks the 4-wide tree or the
+// 64-wide tree (packet.h) as one packet, or every lane walks the 4-wide tree
+// with its own ray and an LDS stack per lane.
+enum UnitTraversal : int { kUnitPacket = 0, kUnitPacketWide = 1, kUnitPerRay = 2 };
 
 // Work counters a launch needs at U.queue: one per slice of the unit range.
 constexpr int kQueueWords = 8;
@@ -128,10 +128,9 @@ void set_split_launches(bool on);
 int render_units_capacity(const DeviceScene& scene, const UnitLaunch& U);
 
 // Traversal of eye rays in renderFrame and the batch paths: 0 = one ray per
-// lane, 1 = wave packets, 2 = wave packets reading nodes and triangles
-// through the scalar unit (UnitTraversal kUnitPerRay / kUnitPacket /
-// kUnitPacketScalar).
-enum TraceMode : int { kTracePerRay = 0, kTracePacket = 1, kTracePacketScalar = 2 };
+// lane, 1 = wave packets on the 4-wide tree, 2 = wave packets on the 64-wide
+// tree (UnitTraversal kUnitPerRay / kUnitPacket / kUnitPacketWide).
+enum TraceMode : int { kTracePerRay = 0, kTracePacket = 1, kTracePacketWide = 2 };
 void set_trace_mode(int mode);
 int trace_mode();
 int unit_traversal_of(int trace_mode);

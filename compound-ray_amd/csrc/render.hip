@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <string>
 
+#include "packet.h"
 #include "render.h"
 
 namespace eye {
@@ -24,6 +25,7 @@ struct SceneView {
   const float4* cols;
   const uint32_t* texels;
   const TexView* textures;
+  WideTree wide;
   int node_count;
   int sky_mode;
   uint32_t* fault;   // host-visible word set when a packet traversal is entered by a partial wave
@@ -36,60 +38,23 @@ SceneView view_of(const DeviceScene& s) {
   v.cols = s.cols;
   v.texels = s.texels;
   v.textures = s.textures;
+  float ext = 0.0f;
+  for (int a = 0; a < 3; ++a) ext = std::max(ext, s.centroid_hi[a] - s.centroid_lo[a]);
+  v.wide = WideTree{s.wide_nodes, s.wide_tris, s.wide_root, s.wide_stack, ext * kPacketSpread, 4.0f * s.wide_radius};
   v.node_count = s.node_count;
   v.sky_mode = s.sky_mode;
   v.fault = s.fault;
   return v;
 }
 
-struct Hit {
-  float t, b1, b2;
-  uint32_t k;   // sorted triangle position
-  uint32_t id;  // original triangle id, 0xffffffff for a miss
-  float det;    // during traversal b1, b2 hold V, W of the closest hit and det its
-                // determinant; finish_hit divides them (b1 = V / det, b2 = W / det)
-};
-
-__device__ __forceinline__ void finish_hit(Hit& h) {
-  if (h.id != 0xffffffffu) {
-    h.b1 = h.b1 / h.det;
-    h.b2 = h.b2 / h.det;
-  }
-}
-
-// Pointers into the constant address space: wave-uniform loads through them
-// become scalar (SMEM) loads, fetched once per wave into SGPRs.  Only used for
-// data no kernel writes while it is read (nodes, triangles).
-typedef float nf4 __attribute__((ext_vector_type(4)));
-typedef int ni4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(4))) const nf4 kf4;
-typedef __attribute__((address_space(4))) const ni4 ki4;
-
-struct UniformPtr {   // float4 array read through the constant address space
-  const void* p;
-};
-struct VaryingPtr {   // float4 array read with per-lane (vector) loads
-  const float4* p;
-};
-__device__ __forceinline__ float4 load4(UniformPtr b, size_t i) {
-  const nf4 v = ((const kf4*)b.p)[i];
-  return make_float4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ float4 load4(VaryingPtr b, size_t i) { return b.p[i]; }
-__device__ __forceinline__ int4 load_int4_uniform(const void* p, size_t i) {
-  const ni4 v = ((const ki4*)p)[i];
-  return make_int4(v.x, v.y, v.z, v.w);
-}
-
-template <typename P4>
-__device__ __forceinline__ void test_leaf(P4 tris, int32_t code, const RayPre& rp, Hit& h) {
+__device__ __forceinline__ void test_leaf(const float4* tris, int32_t code, const RayPre& rp, Hit& h) {
   const uint32_t first = leaf_first(code);
   const uint32_t cnt = leaf_count(code);
   for (uint32_t q = 0; q < cnt; ++q) {
     const uint32_t k = first + q;
-    const float4 a = load4(tris, 3 * (size_t)k + 0);
-    const float4 b = load4(tris, 3 * (size_t)k + 1);
-    const float4 c = load4(tris, 3 * (size_t)k + 2);
+    const float4 a = tris[3 * (size_t)k + 0];
+    const float4 b = tris[3 * (size_t)k + 1];
+    const float4 c = tris[3 * (size_t)k + 2];
     float t, vv, ww, det;
     if (intersect_triangle_raw(rp, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), v3(c.x, c.y, c.z), &t, &vv, &ww, &det)) {
       const uint32_t id = __float_as_uint(a.w);
@@ -104,8 +69,6 @@ __device__ __forceinline__ void test_leaf(P4 tris, int32_t code, const RayPre& r
     }
   }
 }
-
-__device__ __forceinline__ float lane_f(int v, int l) { return __int_as_float(__builtin_amdgcn_readlane(v, l)); }
 
 // A wave-uniform leaf (packet traversal, every lane of the wave executing).
 // Triangle records are 12 dwords (three float4: vertex xyz, and the original
@@ -211,7 +174,7 @@ __device__ __forceinline__ void closest_hit_impl(const SceneView& S, const RayPr
         if (c == kChildEmpty || !(te[s] < INFINITY)) continue;
         if (child_is_leaf(c)) {
           if (kStats) *tris_tested += leaf_count(c);
-          test_leaf(VaryingPtr{S.tris}, c, rp, h);
+          test_leaf(S.tris, c, rp, h);
         } else {
           sorted_insert(it, ic, ni, te[s], c);
           ++ni;
@@ -289,9 +252,10 @@ __device__ __forceinline__ void locate_ray(const EyeLaunch& L, uint64_t r, int* 
 }
 
 // ---------------------------------------------------------------------------
-// Wave-packet traversal.  The 64 rays of a wave are samples of one or two
-// neighbouring ommatidia: nearly the same origin and direction.  The wave
-// walks the BVH together: the node index is wave-uniform (scalar loads), each
+// Wave-packet traversal of the 4-wide tree (trace mode 1; trace mode 2, the
+// default, walks the 64-wide tree, packet.h).  The 64 rays of a wave are
+// samples of one or two neighbouring ommatidia: nearly the same origin and
+// direction.  The wave walks the BVH together: the node index is wave-uniform, each
 // lane tests the children against its own ray and closest hit, a child is
 // entered when any lane's ray enters it, and every active lane tests the
 // triangles of an entered leaf.  Each lane still computes the exact
@@ -320,7 +284,7 @@ __device__ __forceinline__ int stack_top(int s0, int s1, int sp) {
 // One node of a packet step: tests its leaf children (every lane, against
 // its own ray) and appends the internal children that any lane enters to
 // ic / ik (child, ordering key).
-template <bool kParallel, bool kScalar>
+template <bool kParallel>
 __device__ __forceinline__ void packet_visit(const SceneView& S, const RayPre& rp, bool active, int node, Hit& h,
                                              int (&ic)[kBvhWidth], uint32_t (&ik)[kBvhWidth], int& ni,
                                              uint32_t& tris) {
@@ -329,18 +293,9 @@ __device__ __forceinline__ void packet_visit(const SceneView& S, const RayPre& r
   const float limit = h.t * kCullSlack;
 #pragma unroll
   for (int hf = 0; hf < kBvhHalves; ++hf) {
-    float4 lx, hx, ly, hy, lz, hz;
-    int4 ch;
-    if (kScalar) {
-      const UniformPtr np{S.nodes + node};
-      lx = load4(np, 8 * hf + 0); hx = load4(np, 8 * hf + 1); ly = load4(np, 8 * hf + 2);
-      hy = load4(np, 8 * hf + 3); lz = load4(np, 8 * hf + 4); hz = load4(np, 8 * hf + 5);
-      ch = load_int4_uniform(np.p, 8 * hf + 6);
-    } else {
-      const float4* np = reinterpret_cast<const float4*>(S.nodes + node) + 8 * hf;
-      lx = np[0]; hx = np[1]; ly = np[2]; hy = np[3]; lz = np[4]; hz = np[5];
-      ch = reinterpret_cast<const int4*>(np)[6];
-    }
+    const float4* np = reinterpret_cast<const float4*>(S.nodes + node) + 8 * hf;
+    const float4 lx = np[0], hx = np[1], ly = np[2], hy = np[3], lz = np[4], hz = np[5];
+    const int4 ch = reinterpret_cast<const int4*>(np)[6];
     const float slo_x[kHalfWidth] = {lx.x, lx.y, lx.z, lx.w}, shi_x[kHalfWidth] = {hx.x, hx.y, hx.z, hx.w};
     const float slo_y[kHalfWidth] = {ly.x, ly.y, ly.z, ly.w}, shi_y[kHalfWidth] = {hy.x, hy.y, hy.z, hy.w};
     const float slo_z[kHalfWidth] = {lz.x, lz.y, lz.z, lz.w}, shi_z[kHalfWidth] = {hz.x, hz.y, hz.z, hz.w};
@@ -357,10 +312,7 @@ __device__ __forceinline__ void packet_visit(const SceneView& S, const RayPre& r
       if (child_is_leaf(c)) {
         tris += leaf_count(c);
         // inactive lanes test a dummy ray whose result is discarded
-        if (kScalar)
-          test_leaf(UniformPtr{S.tris}, c, rp, h);
-        else
-          test_leaf_wave(S.tris, c, rp, h);
+        test_leaf_wave(S.tris, c, rp, h);
       } else {
         // order key: the entry distance of the first lane that enters the child
         const uint64_t m = __ballot(mine);
@@ -375,7 +327,7 @@ __device__ __forceinline__ void packet_visit(const SceneView& S, const RayPre& r
 
 // steps / tris count the packet's node visits and the triangles of the leaves
 // it enters (wave-uniform: what the wave fetches from memory).
-template <bool kParallel, bool kScalar>
+template <bool kParallel>
 __device__ __forceinline__ void closest_hit_packet_impl(const SceneView& S, const RayPre& rp, bool active, Hit& h,
                                                         uint32_t& steps, uint32_t& tris) {
   int sp = 0;
@@ -388,7 +340,7 @@ __device__ __forceinline__ void closest_hit_packet_impl(const SceneView& S, cons
     int ic[kBvhWidth];
     uint32_t ik[kBvhWidth];
     ++steps;
-    packet_visit<kParallel, kScalar>(S, rp, active, node, h, ic, ik, ni, tris);
+    packet_visit<kParallel>(S, rp, active, node, h, ic, ik, ni, tris);
     if (ni == 0) {
       if (sp == 0) break;
       --sp;
@@ -408,7 +360,6 @@ __device__ __forceinline__ void closest_hit_packet_impl(const SceneView& S, cons
   }
 }
 
-template <bool kScalar = false>
 __device__ __forceinline__ void closest_hit_packet(const SceneView& S, const RayPre& rp, bool active, Hit& h,
                                                    uint32_t& steps, uint32_t& tris) {
   h.t = rp.tmax;
@@ -425,10 +376,23 @@ __device__ __forceinline__ void closest_hit_packet(const SceneView& S, const Ray
     return;
   }
   if (__ballot(active && rp.par != 0) != 0ull)
-    closest_hit_packet_impl<true, kScalar>(S, rp, active, h, steps, tris);
+    closest_hit_packet_impl<true>(S, rp, active, h, steps, tris);
   else
-    closest_hit_packet_impl<false, kScalar>(S, rp, active, h, steps, tris);
+    closest_hit_packet_impl<false>(S, rp, active, h, steps, tris);
   finish_hit(h);
+}
+
+// The closest hits of a wave's rays by packet traversal kTrav; lds: the
+// block's dynamic LDS (wide walk: a stack per wave).
+template <int kTrav>
+__device__ __forceinline__ void packet_hits(const SceneView& S, const Ray& ray, const RayPre& rp, bool active,
+                                            uint32_t* lds, Hit& h, uint32_t& steps, uint32_t& tris) {
+  if (kTrav == kUnitPacketWide) {
+    uint2* stack = reinterpret_cast<uint2*>(lds) + (size_t)(threadIdx.x >> 6) * (size_t)S.wide.stack;
+    closest_hit_wide(S.wide, ray, rp, active, stack, S.fault, h, steps, tris);
+  } else {
+    closest_hit_packet(S, rp, active, h, steps, tris);
+  }
 }
 
 // The value of lane (lane ^ M), M a power of two below 64, without an
@@ -676,7 +640,7 @@ __global__ __launch_bounds__(kTraceThreads, kTrav == kUnitPerRay ? 4 : 6) void k
           h.b1 = h.b2 = 0.0f;
           if (active) closest_hit(S, rp, lane_stack, (int)blockDim.x, h);
         } else {
-          closest_hit_packet<kTrav == kUnitPacketScalar>(S, rp, active, h, w_steps, w_tris);
+          packet_hits<kTrav>(S, ray, rp, active, unit_lds, h, w_steps, w_tris);
         }
         if (active) {
           const V3 c = shade(S, h, ray.dx, ray.dy, ray.dz);
@@ -863,16 +827,14 @@ __global__ __launch_bounds__(kTraceThreads, 5) void k_render_chunks(SceneView S,
 // between the ray generation and the chunk store, which keeps register use
 // low (more resident waves).  Same per-lane chunk values, completion
 // counters and last-wave reduction as k_render_chunks (no statistics).
-template <bool kSamples, bool kScalar, bool kSplit>
+template <bool kSamples, int kTrav, bool kSplit>
 __global__ __launch_bounds__(kTraceThreads, 6) void k_render_tasks(SceneView S, UnitLaunch U, int chunks) {
+  extern __shared__ uint32_t task_lds[];
   const int lane = threadIdx.x & 63;
   const uint64_t units = (uint64_t)U.pose_count * (uint64_t)U.omm_count;
   const uint64_t tasks = units * (uint64_t)chunks;
-  // With vector node loads the task, unit and output indices go to scalar
-  // registers (the wave index read once as uniform), which keeps the split
-  // variant from spilling; the scalar-load traversal needs those registers
-  // for node words and keeps the indices in vector registers.
-  const uint32_t wave = kScalar ? (threadIdx.x >> 6) : (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  // the wave index read once as uniform: task, unit and output indices go to scalar registers
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const uint64_t wv = (uint64_t)xcd_logical_block(blockIdx.x, gridDim.x) * (kTraceThreads / 64) + (uint64_t)wave;
   // With a long-task split the first kSplitSubWaves waves trace the listed
   // tasks: 4 waves per tier-0 task (wave w: part w % 4 of tier-0 task w / 4),
@@ -949,7 +911,7 @@ __global__ __launch_bounds__(kTraceThreads, 6) void k_render_tasks(SceneView S, 
   }
   Hit h;
   uint32_t w_steps = 0, w_tris = 0;
-  closest_hit_packet<kScalar>(S, rp, mine, h, w_steps, w_tris);
+  packet_hits<kTrav>(S, ray, rp, mine, task_lds, h, w_steps, w_tris);
   if (U.packet_counts && lane == 0) {
     atomicAdd(U.packet_counts, (unsigned long long)w_steps);
     atomicAdd(U.packet_counts + 1, (unsigned long long)w_tris);
@@ -997,15 +959,17 @@ __global__ __launch_bounds__(kTraceThreads, 6) void k_render_tasks(SceneView S, 
 // Failure-handling probe of the packet traversal's partial-wave guard: one
 // wave traces 64 rays, lanes at or above active_lanes skip the call (their
 // ids stay 0xfffffffe).
+template <int kTrav>
 __global__ __launch_bounds__(64) void k_packet_guard_probe(SceneView S, const Ray* __restrict__ rays,
                                                            int active_lanes, int32_t* __restrict__ ids) {
+  extern __shared__ uint32_t probe_lds[];
   const int lane = (int)(threadIdx.x & 63);
   Hit h;
   h.id = 0xfffffffeu;
   if (lane < active_lanes) {
-    const RayPre rp = precompute_ray(rays[lane]);
+    const Ray ray = rays[lane];
     uint32_t steps = 0, tris = 0;
-    closest_hit_packet<false>(S, rp, true, h, steps, tris);
+    packet_hits<kTrav>(S, ray, precompute_ray(ray), true, probe_lds, h, steps, tris);
   }
   ids[lane] = (int32_t)h.id;
 }
@@ -1244,7 +1208,7 @@ size_t stack_bytes(const DeviceScene& s) {
 
 }  // namespace
 
-static int g_trace_mode = kTracePacketScalar;
+static int g_trace_mode = kTracePacketWide;
 static const char* g_last_kernel = "";
 static bool g_split = true;
 
@@ -1310,19 +1274,26 @@ static int device_cus() {
   return cus;
 }
 
-static size_t units_lds_bytes(const DeviceScene& scene, int traversal) {
+// Dynamic LDS of a block of `waves` waves: a stack column per lane (per ray) or
+// per wave (wide packets).
+static size_t units_lds_bytes(const DeviceScene& scene, int traversal, int waves = kTraceThreads / 64) {
+  if (traversal == kUnitPacketWide) return sizeof(uint2) * (size_t)std::max(scene.wide_stack, 1) * (size_t)waves;
   return traversal == kUnitPerRay ? stack_bytes(scene) : 0;
 }
 
-// Packets keep their traversal stack in VGPR lanes (kPacketStackMax entries);
-// a deeper BVH takes the per-ray traversal, whose stacks live in LDS.
+// The wide walk's LDS stacks hold kWideStackMax entries and the 4-wide packets'
+// stack, in VGPR lanes, kPacketStackMax: a deeper tree (or no wide tree) takes
+// the next of them, at last the per-ray traversal.
 static int effective_traversal(const DeviceScene& scene, int traversal) {
+  if (traversal == kUnitPacketWide && scene.node_count > 0 &&
+      (!scene.wide_nodes || scene.wide_stack > kWideStackMax))
+    traversal = kUnitPacket;
   return traversal != kUnitPerRay && scene.stack_bound > kPacketStackMax ? (int)kUnitPerRay : traversal;
 }
 
 static const void* units_kernel_of(const UnitLaunch& U) {
   if (U.traversal == kUnitPerRay) return units_kernel_variant<kUnitPerRay>(U);
-  if (U.traversal == kUnitPacketScalar) return units_kernel_variant<kUnitPacketScalar>(U);
+  if (U.traversal == kUnitPacketWide) return units_kernel_variant<kUnitPacketWide>(U);
   return units_kernel_variant<kUnitPacket>(U);
 }
 
@@ -1403,14 +1374,15 @@ bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipSt
       }
       const uint64_t waves = tasks + (T.split_flag ? (uint64_t)kSplitSubWaves : 0u);
       const dim3 grid((unsigned)((waves + (kTraceThreads / 64) - 1) / (kTraceThreads / 64))), block(kTraceThreads);
-      const bool scalar = U.traversal == kUnitPacketScalar;
+      const bool wide = U.traversal == kUnitPacketWide;
+      constexpr int kW = kUnitPacketWide, kP = kUnitPacket;
       // the variant without the split's code keeps the registers of the plain task kernel
-      auto kernel = U.samples ? (scalar ? k_render_tasks<true, true, false> : k_render_tasks<true, false, false>)
-                              : (scalar ? k_render_tasks<false, true, false> : k_render_tasks<false, false, false>);
+      auto kernel = U.samples ? (wide ? k_render_tasks<true, kW, false> : k_render_tasks<true, kP, false>)
+                              : (wide ? k_render_tasks<false, kW, false> : k_render_tasks<false, kP, false>);
       if (T.split_cost)
-        kernel = U.samples ? (scalar ? k_render_tasks<true, true, true> : k_render_tasks<true, false, true>)
-                           : (scalar ? k_render_tasks<false, true, true> : k_render_tasks<false, false, true>);
-      hipLaunchKernelGGL(kernel, grid, block, 0, stream, v, T, (int)chunks);
+        kernel = U.samples ? (wide ? k_render_tasks<true, kW, true> : k_render_tasks<true, kP, true>)
+                           : (wide ? k_render_tasks<false, kW, true> : k_render_tasks<false, kP, true>);
+      hipLaunchKernelGGL(kernel, grid, block, lds, stream, v, T, (int)chunks);
       g_last_kernel = "k_render_tasks";
       return check_launch("render_tasks", err);
     }
@@ -1445,8 +1417,8 @@ bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipSt
   hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, stream, G.queue, (uint32_t)kQueueWords, 0u);
   if (G.traversal == kUnitPerRay)
     launch_units_variant<kUnitPerRay>(G, v, blocks, lds, stream);
-  else if (G.traversal == kUnitPacketScalar)
-    launch_units_variant<kUnitPacketScalar>(G, v, blocks, lds, stream);
+  else if (G.traversal == kUnitPacketWide)
+    launch_units_variant<kUnitPacketWide>(G, v, blocks, lds, stream);
   else
     launch_units_variant<kUnitPacket>(G, v, blocks, lds, stream);
   g_last_kernel = "k_render_units";
@@ -1459,10 +1431,10 @@ void set_split_launches(bool on) { g_split = on; }
 void set_trace_mode(int mode) { g_trace_mode = mode; }
 int trace_mode() { return g_trace_mode; }
 int unit_traversal_of(int mode) {
-  return mode == kTracePerRay ? kUnitPerRay : mode == kTracePacketScalar ? kUnitPacketScalar : kUnitPacket;
+  return mode == kTracePerRay ? kUnitPerRay : mode == kTracePacketWide ? kUnitPacketWide : kUnitPacket;
 }
 int trace_mode_of(int traversal) {
-  return traversal == kUnitPerRay ? kTracePerRay : traversal == kUnitPacketScalar ? kTracePacketScalar : kTracePacket;
+  return traversal == kUnitPerRay ? kTracePerRay : traversal == kUnitPacketWide ? kTracePacketWide : kTracePacket;
 }
 
 bool launch_copy_probe(const float4* src, float4* dst, size_t n, hipStream_t stream, std::string* err) {
@@ -1537,11 +1509,18 @@ bool launch_generate_rays(const EyeLaunch& L, Ray* rays, hipStream_t stream, std
 
 bool launch_packet_guard_probe(const DeviceScene& scene, const Ray* rays, int active_lanes, int32_t* ids,
                                hipStream_t stream, std::string* err) {
-  if (scene.stack_bound > kPacketStackMax) {
+  const int trav = effective_traversal(scene, kUnitPacketWide);
+  if (trav == kUnitPerRay) {
     if (err) *err = "packet probe: BVH too deep for the packet traversal";
     return false;
   }
-  hipLaunchKernelGGL(k_packet_guard_probe, dim3(1), dim3(64), 0, stream, view_of(scene), rays, active_lanes, ids);
+  const size_t lds = units_lds_bytes(scene, trav, 1);
+  if (trav == kUnitPacketWide)
+    hipLaunchKernelGGL(k_packet_guard_probe<kUnitPacketWide>, dim3(1), dim3(64), lds, stream, view_of(scene), rays,
+                       active_lanes, ids);
+  else
+    hipLaunchKernelGGL(k_packet_guard_probe<kUnitPacket>, dim3(1), dim3(64), lds, stream, view_of(scene), rays,
+                       active_lanes, ids);
   return check_launch("packet_guard_probe", err);
 }
 

@@ -272,8 +272,8 @@ int setSceneLeafSize(int leafSize);
  * a later render can add samples independent of an earlier one. */
 void setCurrentEyeSampleBase(uint32_t base);
 /* Traversal strategy of eye rays: 0 = one ray per lane (own LDS stack),
- * 1 = wave packets, 2 = wave packets reading nodes and triangles through the
- * scalar unit (default).  Results are identical; only speed differs.
+ * 1 = wave packets on the 4-wide BVH, 2 = wave packets on a 64-wide tree of
+ * the same triangles (default).  Results are identical; only speed differs.
  * autotuneRenderBatch sets it to the tuned winner. */
 void setTraversalMode(int mode);
 /* Keep the per-sample records of renderFrame for getCurrentEyeSamples (off by
@@ -319,8 +319,8 @@ void setBatchAutotune(int enabled);
 int setAutotuneCacheFile(const char* path);
 /* Times every candidate shape on (a sample of) these poses and installs the
  * fastest as the shape of all later unit launches.  trials receives rows of
- * 4 floats (units per grab, blocks, traversal: 0 packet, 1 packet with scalar
- * loads, 2 per-ray; ms); returns the number of candidates, -1 on error. */
+ * 4 floats (units per grab, blocks, traversal: 0 packet, 1 packet on the
+ * 64-wide tree, 2 per-ray; ms); returns the number of candidates, -1 on error. */
 int autotuneRenderBatch(const float* poses, size_t poseCount, int repeats, float* trials, size_t maxTrials);
 
 /* Bandwidth reference for profiling: copies `bytes` (rounded down to 16-byte
