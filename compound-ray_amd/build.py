@@ -34,7 +34,6 @@ SOURCES = [
     "mlp.hip",
     "adaptive.hip",
     "knn.cpp",
-    "noalloc.hip",
     "eye_renderer.cpp",
 ]
 

@@ -94,7 +94,6 @@ class AdaptiveRenderer {
   float* d_part_ = nullptr;       // partial sums of the allocation
   size_t part_cap_ = 0;
   float* d_sqrt_ = nullptr;       // per pose: sum of sqrt(n_req)
-  uint32_t* d_queue_ = nullptr;
   size_t units_cap_ = 0;
   hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
   hipEvent_t ev_stage_[3] = {nullptr, nullptr, nullptr};   // after the pilot, the allocation, the top-up

@@ -214,7 +214,7 @@ bool ok_launch(const char* what, std::string* err) {
 
 void AdaptiveRenderer::release() {
   for (void* p : {(void*)d_poses_, (void*)d_col_a_, (void*)d_col_b_, (void*)d_final_, (void*)d_stats_, (void*)d_feat_,
-                  (void*)d_pred_, (void*)d_counts_, (void*)d_extra_, (void*)d_total_, (void*)d_queue_,
+                  (void*)d_pred_, (void*)d_counts_, (void*)d_extra_, (void*)d_total_,
                   (void*)d_part_, (void*)d_sqrt_})
     if (p) (void)hipFree(p);
   d_poses_ = nullptr;
@@ -222,7 +222,7 @@ void AdaptiveRenderer::release() {
   part_cap_ = 0;
   d_col_a_ = d_col_b_ = d_final_ = d_stats_ = nullptr;
   d_feat_ = d_pred_ = nullptr;
-  d_counts_ = d_extra_ = d_queue_ = nullptr;
+  d_counts_ = d_extra_ = nullptr;
   d_total_ = nullptr;
   poses_cap_ = units_cap_ = 0;
   if (ev0_) (void)hipEventDestroy(ev0_);
@@ -241,7 +241,7 @@ bool AdaptiveRenderer::ensure(size_t poses, size_t units, std::string* err) {
     if (err) *err = "adaptive: event creation failed";
     return false;
   }
-  if (!d_total_ && (!grow(&d_total_, 1, err) || !grow(&d_queue_, kQueueWords, err))) return false;
+  if (!d_total_ && !grow(&d_total_, 1, err)) return false;
   if (poses > poses_cap_) {
     if (!grow(&d_poses_, poses, err) || !grow(&d_sqrt_, poses, err)) return false;
     poses_cap_ = poses;
@@ -302,7 +302,6 @@ bool AdaptiveRenderer::render(const DeviceScene& scene, UnitLaunch U, const std:
   A.colours = d_col_a_;
   A.stats = d_stats_;
   A.samples = nullptr;
-  A.queue = d_queue_;
   // Grab size chosen per pass (0: automatic).  A tuned size comes from uniform
   // batches; a grab of few pilot units would leave most of the wave's lanes idle.
   // Pilot grabs of at most 8 units (one 64-lane round of 8-sample units):
@@ -421,7 +420,6 @@ bool AdaptiveRenderer::training_set(const DeviceScene& scene, UnitLaunch U, cons
   A.colours = d_col_a_;
   A.stats = d_stats_;
   A.samples = nullptr;
-  A.queue = d_queue_;
   A.units_per_grab = 0;  // automatic, as in render()
   A.auto_grab_max = 8;
   if (!launch_render_units(scene, A, stream, err)) return false;

@@ -25,15 +25,6 @@ bool grow(T** p, size_t* cap, size_t n, std::string* err) {
   return true;
 }
 
-bool same_launch(const UnitLaunch& a, const UnitLaunch& b) {
-  return a.omms == b.omms && a.omm_count == b.omm_count && a.poses == b.poses && a.pose_count == b.pose_count &&
-         a.pose_base == b.pose_base && a.seed == b.seed && a.eye == b.eye && a.frame == b.frame && a.spp == b.spp &&
-         a.omm_counts == b.omm_counts && a.unit_counts == b.unit_counts && a.sample_base == b.sample_base &&
-         a.order == b.order && a.colours == b.colours && a.stats == b.stats && a.samples == b.samples &&
-         a.sample_offsets == b.sample_offsets && a.queue == b.queue && a.units_per_grab == b.units_per_grab &&
-         a.auto_grab_max == b.auto_grab_max && a.blocks == b.blocks && a.traversal == b.traversal &&
-         a.packet_counts == b.packet_counts;
-}
 }  // namespace
 
 std::vector<LaunchShape> LaunchTuner::candidates(int capacity) {
@@ -117,56 +108,17 @@ bool LaunchTuner::save(const std::string& path, std::string* err) const {
 }
 
 void BatchRenderer::release() {
-  if (exec_) (void)hipGraphExecDestroy(exec_);
-  if (graph_) (void)hipGraphDestroy(graph_);
-  exec_ = nullptr;
-  graph_ = nullptr;
   if (d_poses_) (void)hipFree(d_poses_);
   if (d_colours_) (void)hipFree(d_colours_);
-  if (d_queue_) (void)hipFree(d_queue_);
   if (ev0_) (void)hipEventDestroy(ev0_);
   if (ev1_) (void)hipEventDestroy(ev1_);
   d_poses_ = nullptr;
   d_colours_ = nullptr;
-  d_queue_ = nullptr;
   ev0_ = ev1_ = nullptr;
   poses_cap_ = colours_cap_ = 0;
-  g_valid_ = false;
-  g_scene_ = 0;
 }
 
-bool BatchRenderer::build_graph(const DeviceScene& scene, const UnitLaunch& U, hipStream_t stream,
-                                std::string* err) {
-  if (exec_) (void)hipGraphExecDestroy(exec_);
-  if (graph_) (void)hipGraphDestroy(graph_);
-  exec_ = nullptr;
-  graph_ = nullptr;
-  hipError_t e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
-  if (e != hipSuccess) {
-    if (err) *err = std::string("batch: begin capture: ") + hipGetErrorString(e);
-    return false;
-  }
-  std::string lerr;
-  const bool ok = launch_render_units(scene, U, stream, &lerr);
-  e = hipStreamEndCapture(stream, &graph_);
-  if (!ok || e != hipSuccess) {
-    if (err) *err = !ok ? lerr : std::string("batch: end capture: ") + hipGetErrorString(e);
-    if (graph_) (void)hipGraphDestroy(graph_);
-    graph_ = nullptr;
-    return false;
-  }
-  e = hipGraphInstantiate(&exec_, graph_, nullptr, nullptr, 0);
-  if (e != hipSuccess) {
-    if (err) *err = std::string("batch: instantiate: ") + hipGetErrorString(e);
-    return false;
-  }
-  g_launch_ = U;
-  g_valid_ = true;
-  g_scene_ = scene.generation;
-  return true;
-}
-
-bool BatchRenderer::prepare(const UnitLaunch& U, const std::vector<Pose>& poses, hipStream_t stream, bool* realloc,
+bool BatchRenderer::prepare(const UnitLaunch& U, const std::vector<Pose>& poses, hipStream_t stream,
                             std::string* err) {
   const size_t np = poses.size();
   if (!ev0_ && (hipEventCreate(&ev0_) != hipSuccess || hipEventCreate(&ev1_) != hipSuccess)) {
@@ -174,13 +126,8 @@ bool BatchRenderer::prepare(const UnitLaunch& U, const std::vector<Pose>& poses,
     return false;
   }
   const size_t units = np * (size_t)U.omm_count;
-  *realloc = poses_cap_ < np || colours_cap_ < units;
   if (!grow(&d_poses_, &poses_cap_, np, err)) return false;
   if (!grow(&d_colours_, &colours_cap_, units, err)) return false;
-  if (!d_queue_ && hipMalloc(&d_queue_, sizeof(uint32_t) * kQueueWords) != hipSuccess) {
-    if (err) *err = "batch: queue allocation failed";
-    return false;
-  }
   if (hipMemcpyAsync(d_poses_, poses.data(), sizeof(Pose) * np, hipMemcpyHostToDevice, stream) != hipSuccess) {
     if (err) *err = "batch: pose upload failed";
     return false;
@@ -195,13 +142,11 @@ bool BatchRenderer::tune(const DeviceScene& scene, UnitLaunch U, const std::vect
     if (err) *err = "autotune: empty batch";
     return false;
   }
-  bool realloc = false;
-  if (!prepare(U, poses, stream, &realloc, err)) return false;
+  if (!prepare(U, poses, stream, err)) return false;
   U.poses = d_poses_;
   U.pose_count = (int)poses.size();
   U.pose_base = 0;
   U.colours = d_colours_;
-  U.queue = d_queue_;
   U.stats = nullptr;
   U.samples = nullptr;
   const int capacity = render_units_capacity(scene, U);
@@ -239,25 +184,13 @@ bool BatchRenderer::render(const DeviceScene& scene, UnitLaunch U, const std::ve
   *gpu_ms = 0.0;
   if (np == 0) return true;
   const size_t units = np * (size_t)U.omm_count;
-  bool realloc = false;
-  if (!prepare(U, poses, stream, &realloc, err)) return false;
+  if (!prepare(U, poses, stream, err)) return false;
   U.poses = d_poses_;
   U.pose_count = (int)np;
   U.pose_base = 0;
   U.colours = d_colours_;
-  U.queue = d_queue_;
-  if (use_graph_) {
-    if (realloc || !exec_ || !g_valid_ || g_scene_ != scene.generation || !same_launch(U, g_launch_))
-      if (!build_graph(scene, U, stream, err)) return false;
-    (void)hipEventRecord(ev0_, stream);
-    if (hipGraphLaunch(exec_, stream) != hipSuccess) {
-      if (err) *err = "batch: graph launch failed";
-      return false;
-    }
-  } else {
-    (void)hipEventRecord(ev0_, stream);
-    if (!launch_render_units(scene, U, stream, err)) return false;
-  }
+  (void)hipEventRecord(ev0_, stream);
+  if (!launch_render_units(scene, U, stream, err)) return false;
   (void)hipEventRecord(ev1_, stream);
   if (hipEventSynchronize(ev1_) != hipSuccess) {
     if (err) *err = "batch: render failed";

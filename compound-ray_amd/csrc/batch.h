@@ -1,10 +1,9 @@
 // Batched rendering of one eye at many poses (no reference counterpart: the
 // reference renders one pose per renderFrame call, libEyeRenderer.cpp:229-242).
 //
-// All (pose, ommatidium) units of a batch go through one persistent launch of
-// the unit renderer.  The launch sequence (queue reset + render) is captured
-// once into a HIP graph per batch shape and replayed; the launch shape (units
-// per queue grab, blocks) comes from the autotuner when one is attached.
+// All (pose, ommatidium) units of a batch go through one launch of the unit
+// renderer; the launch shape (units per wave, blocks) comes from the autotuner
+// when one is attached.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -20,7 +19,7 @@ namespace eye {
 // Launch shape of the unit renderer.
 struct LaunchShape {
   int units_per_grab = 4;
-  int blocks = 0;  // 0: resident capacity
+  int blocks = 0;  // 0: a wave per grab
   int traversal = 0;  // UnitTraversal
 };
 
@@ -66,26 +65,15 @@ class BatchRenderer {
             hipStream_t stream, std::vector<TuneTrial>* trials, LaunchShape* best, std::string* err);
   // Device colours of the last batch, [pose][omm] float4.
   const float4* colours() const { return d_colours_; }
-  void set_use_graph(bool on) { use_graph_ = on; }
   void release();
 
  private:
-  bool build_graph(const DeviceScene& scene, const UnitLaunch& U, hipStream_t stream, std::string* err);
-  bool prepare(const UnitLaunch& U, const std::vector<Pose>& poses, hipStream_t stream, bool* realloc,
-               std::string* err);
+  bool prepare(const UnitLaunch& U, const std::vector<Pose>& poses, hipStream_t stream, std::string* err);
   Pose* d_poses_ = nullptr;
   size_t poses_cap_ = 0;
   float4* d_colours_ = nullptr;
   size_t colours_cap_ = 0;
-  uint32_t* d_queue_ = nullptr;
   hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
-  bool use_graph_ = true;
-  hipGraph_t graph_ = nullptr;
-  hipGraphExec_t exec_ = nullptr;
-  // shape the captured graph was built for
-  uint64_t g_scene_ = 0;  // generation of the scene the graph was captured on
-  UnitLaunch g_launch_;
-  bool g_valid_ = false;
 };
 
 }  // namespace eye

@@ -22,7 +22,6 @@
 #include "device_scene.h"
 #include "knn.h"
 #include "mlp.h"
-#include "noalloc.h"
 #include "render.h"
 #include "projection.h"
 #include "scene_loader.h"
@@ -145,7 +144,6 @@ struct State {
   Mlp mlp;
   AdaptiveRenderer adaptive;
   bool record_samples = false;   // keep per-sample records of renderFrame
-  uint32_t* d_queue = nullptr;   // work counter of the unit renderer
   int units_per_grab = 0;        // 0: automatic
   int unit_blocks = 0;           // 0: automatic
   bool autotune = false;         // tune renderPoseBatch's launch shape per workload
@@ -183,12 +181,9 @@ void ensure_hip() {
   const hipError_t e = hipGetDeviceCount(&count);
   if (e != hipSuccess || count == 0) throw std::runtime_error("no HIP device available");
   hip_check(hipSetDevice(0), "hipSetDevice");
-  std::string serr;
-  if (!no_alloc_scratch_init(0, &serr)) throw std::runtime_error(serr);
   hip_check(hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking), "hipStreamCreate");
   hip_check(hipMalloc(&s.d_pose, sizeof(Pose)), "hipMalloc pose");
   hip_check(hipMalloc(&s.d_stats, sizeof(unsigned long long) * 4), "hipMalloc stats");
-  hip_check(hipMalloc(&s.d_queue, sizeof(uint32_t) * kQueueWords), "hipMalloc queue");
   hip_check(hipMalloc(&s.d_packet_counts, sizeof(unsigned long long) * 2), "hipMalloc packet counts");
   hip_check(hipMemset(s.d_packet_counts, 0, sizeof(unsigned long long) * 2), "clear packet counts");
   for (hipEvent_t& e : s.ev) hip_check(hipEventCreate(&e), "hipEventCreate");
@@ -424,7 +419,6 @@ UnitLaunch unit_launch_of(EyeState& e, const Pose* d_poses, int pose_count) {
   U.spp = e.spp;
   U.omm_counts = e.counts.empty() ? nullptr : e.d_counts;
   U.colours = e.d_colours;
-  U.queue = s.d_queue;
   U.units_per_grab = s.units_per_grab;
   U.blocks = s.unit_blocks;
   U.traversal = unit_traversal_of(trace_mode());
@@ -1338,18 +1332,15 @@ int renderPoseBatchInto(const float* devPoses, size_t poseCount, float* devColou
   if ((reinterpret_cast<uintptr_t>(devPoses) & 3u) != 0 || (reinterpret_cast<uintptr_t>(devColours) & 15u) != 0)
     throw std::runtime_error("renderPoseBatchInto: poses must be 4-byte and colours 16-byte aligned");
   const uint64_t units = (uint64_t)poseCount * (uint64_t)e->omms.size();
-  if (poseCount > (size_t)INT32_MAX || units > kNoAllocMaxUnits)
+  if (poseCount > (size_t)INT32_MAX || units > kMaxLaunchUnits)
     throw std::runtime_error("renderPoseBatchInto: " + std::to_string(units) + " units exceed the maximum of " +
-                             std::to_string(kNoAllocMaxUnits) + " per call");
+                             std::to_string(kMaxLaunchUnits) + " per call");
   if (e->device_dirty())
     throw std::runtime_error(
         "renderPoseBatchInto: the current eye's ommatidia or sample counts changed since they were last uploaded; "
         "render the eye once with renderFrame or renderPoseBatch first (those calls may allocate)");
-  uint32_t* scratch = no_alloc_scratch(0);
-  if (!scratch) throw std::runtime_error("renderPoseBatchInto: fixed scratch not initialised");
   UnitLaunch U = unit_launch_of(*e, reinterpret_cast<const Pose*>(devPoses), (int)poseCount);
   U.colours = reinterpret_cast<float4*>(devColours);
-  U.queue = scratch;
   std::string err;
   if (!launch_render_units(s.scene, U, stream ? static_cast<hipStream_t>(stream) : s.stream, &err))
     throw std::runtime_error(err);

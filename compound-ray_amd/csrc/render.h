@@ -47,11 +47,11 @@ constexpr uint64_t split_buffer_words(uint64_t tasks) {
   return 2 * tasks + (uint64_t)kSplitListMax + kSplitCountWords + kSplitSubMax;
 }
 
-// Persistent ommatidium-unit renderer.  A unit is one ommatidium at one pose;
-// waves take units from a work queue (`units_per_grab` at a time), trace a
-// unit's samples 64 at a time as one wave packet and reduce them in registers
-// in the canonical order (lane l sums samples l, l+64, ... then an xor
-// butterfly), so no per-sample buffer is needed.
+// Ommatidium-unit renderer.  A unit is one ommatidium at one pose; a wave
+// renders `units_per_grab` consecutive units, traces a unit's samples 64 at a
+// time as one wave packet and reduces them in registers in the canonical
+// order (lane l sums samples l, l+64, ... then an xor butterfly), so no
+// per-sample buffer is needed.
 struct UnitLaunch {
   const Ommatidium* omms = nullptr;
   int omm_count = 0;
@@ -69,7 +69,6 @@ struct UnitLaunch {
                                         //   (mean inverse depth, its variance, 0, 0)
   float4* samples = nullptr;            // nullable: per-sample (r, g, b, t or -1)
   const uint64_t* sample_offsets = nullptr;  // first sample record of each unit
-  uint32_t* queue = nullptr;            // device work counters (kQueueWords)
   // Optional scratch for split launches (uniform sample counts and few
   // units): each unit's 64-sample chunks go to different waves; per-lane
   // chunk values (1 float4, 3 with stats) and a completion counter per unit.
@@ -94,10 +93,11 @@ struct UnitLaunch {
   uint64_t split_tasks = 0;
   bool split_plan = false;
   // launch shape (results do not depend on it)
-  int units_per_grab = 0;               // consecutive units a wave takes from the queue (0: chosen
-                                        //   from the launch size, at most auto_grab_max)
+  int units_per_grab = 0;               // consecutive units per wave (0: chosen from the launch
+                                        //   size, at most auto_grab_max)
   int auto_grab_max = 16;
-  int blocks = 0;                       // blocks of 256 threads; 0: every resident slot once
+  int blocks = 0;                       // blocks of 256 threads, which stride over the work; 0: a
+                                        //   wave per grab
   int traversal = 0;                    // UnitTraversal
   // nullable: packet traversals add their node visits ([0]) and the triangles
   // of the leaves they enter ([1]), counted once per wave (measurement runs)
@@ -109,13 +109,12 @@ struct UnitLaunch {
 // with its own ray and an LDS stack per lane.
 enum UnitTraversal : int { kUnitPacket = 0, kUnitPacketWide = 1, kUnitPerRay = 2 };
 
-// Work counters a launch needs at U.queue: one per slice of the unit range.
-constexpr int kQueueWords = 8;
+// Most (pose, ommatidium) units of one launch: their indices are 32-bit.
+constexpr uint64_t kMaxLaunchUnits = 0xffffffffull - 65536ull;
 // Largest grab of the unit renderer: lane g of a wave holds unit g's count.
 constexpr int kMaxUnitsPerGrab = 64;
 
-// Launches the unit renderer with U's launch shape.  The queue counter is
-// cleared by a kernel first.
+// Launches the unit renderer with U's launch shape.
 bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U, hipStream_t stream, std::string* err);
 
 // Name of the kernel the last launch_render_units used (k_render_units or the

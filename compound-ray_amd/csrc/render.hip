@@ -16,7 +16,6 @@ namespace {
 constexpr int kTraceThreads = 256;
 // XCDs of the device: workgroup b runs on XCD b % kXcds, each with its own L2.
 constexpr uint32_t kXcds = 8;
-static_assert(kQueueWords >= (int)kXcds, "one work counter per XCD slice");
 constexpr int kPacketStackMax = 128;  // two VGPRs of 64 lanes
 
 struct SceneView {
@@ -213,17 +212,21 @@ __device__ __forceinline__ void closest_hit(const SceneView& S, const RayPre& rp
   finish_hit(h);
 }
 
-__device__ __forceinline__ V3 shade(const SceneView& S, const Hit& h, float dx, float dy, float dz) {
-  if (h.id == 0xffffffffu) return sky_colour(S.sky_mode, dx, dy, dz);
-  const float4 c0 = S.cols[3 * (size_t)h.k + 0];
-  const float4 c1 = S.cols[3 * (size_t)h.k + 1];
+__device__ __forceinline__ V3 shade(const float4* cols, const uint32_t* texels, const TexView* textures, int sky_mode,
+                                    const Hit& h, float dx, float dy, float dz) {
+  if (h.id == 0xffffffffu) return sky_colour(sky_mode, dx, dy, dz);
+  const float4 c0 = cols[3 * (size_t)h.k + 0];
+  const float4 c1 = cols[3 * (size_t)h.k + 1];
   const uint32_t word = __float_as_uint(c0.w);
   if (colour_mode(word) == kTextureColour) {
     const float uv[6] = {c0.x, c0.y, c0.z, c1.x, c1.y, c1.z};
-    return shade_texture(h.b1, h.b2, uv, S.texels, S.textures[texture_index(word)]);
+    return shade_texture(h.b1, h.b2, uv, texels, textures[texture_index(word)]);
   }
-  const float4 c2 = S.cols[3 * (size_t)h.k + 2];
+  const float4 c2 = cols[3 * (size_t)h.k + 2];
   return shade_hit(h.b1, h.b2, v3(c0.x, c0.y, c0.z), v3(c1.x, c1.y, c1.z), v3(c2.x, c2.y, c2.z), word);
+}
+__device__ __forceinline__ V3 shade(const SceneView& S, const Hit& h, float dx, float dy, float dz) {
+  return shade(S.cols, S.texels, S.textures, S.sky_mode, h, dx, dy, dz);
 }
 
 // Maps a ray number to (pose, ommatidium, sample, samples of that ommatidium).
@@ -426,12 +429,6 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
-__device__ __forceinline__ uint32_t unit_count(const UnitLaunch& U, uint64_t u, int i) {
-  if (U.unit_counts) return U.unit_counts[u];
-  if (U.omm_counts) return U.omm_counts[i];
-  return (uint32_t)U.spp;
-}
-
 // Segmented form of wave_sum: lanes [a, a + seg) with a a multiple of seg
 // (a power of two) sum their values; lane a ends with the total.  For a unit
 // whose samples occupy lanes a .. a + n - 1 (n <= seg, other lanes 0) this is
@@ -452,18 +449,7 @@ __device__ __forceinline__ float segment_sum(float v, int seg) {
   return v;
 }
 
-// Pose, ommatidium and output slot of queue position u.
-// The unit renderer's launches hold fewer than 2^32 units (launch_render_units
-// checks), so its queue positions and output slots are 32-bit.
-__device__ __forceinline__ void locate_unit32(const UnitLaunch& U, uint32_t u, int* p, int* i, uint32_t* out) {
-  const uint32_t n = (uint32_t)U.omm_count;
-  const uint32_t q = u / n;
-  const uint32_t k = u - q * n;
-  *p = (int)q;
-  *i = U.order ? (int)U.order[k] : (int)k;
-  *out = q * n + (uint32_t)*i;
-}
-
+// Pose, ommatidium and output slot of unit u of the processing order.
 __device__ __forceinline__ void locate_unit(const UnitLaunch& U, uint64_t u, int* p, int* i, uint64_t* out) {
   *p = (int)(u / (uint64_t)U.omm_count);
   const int k = (int)(u - (uint64_t)*p * (uint64_t)U.omm_count);
@@ -501,130 +487,180 @@ __device__ __forceinline__ int pow2_at_least(uint32_t n) {
   return s;
 }
 
-// Persistent unit renderer.  A wave takes units_per_grab consecutive units
-// from the queue and renders them in rounds: a unit of more than 32 samples
+// Workgroups are handed to the 8 XCDs round-robin (block b to XCD b % 8),
+// and each XCD has its own L2.  Logical blocks are therefore dealt to XCDs in
+// runs of kXcdRun consecutive blocks: the processing order is the Morton order of the
+// ommatidial axes, so an XCD's resident waves look in neighbouring directions
+// and share BVH nodes in its L2, while runs still alternate between XCDs so
+// that each gets its share of costly directions.  The mapping is a
+// bijection, so results do not depend on it.
+constexpr uint32_t kXcdRun = 16;
+
+__device__ __forceinline__ uint32_t xcd_run_block(uint32_t b, uint32_t blocks, uint32_t run) {
+  const uint32_t span = kXcds * run;
+  if (b >= (blocks / span) * span) return b;
+  const uint32_t x = b % kXcds, j = b / kXcds;
+  return ((j / run) * kXcds + x) * run + j % run;
+}
+__device__ __forceinline__ uint32_t xcd_logical_block(uint32_t b, uint32_t blocks) {
+  return xcd_run_block(b, blocks, kXcdRun);
+}
+
+// Unit renderer.  A wave takes units_per_grab consecutive units of the
+// processing order and renders them in rounds: a unit of more than 32 samples
 // fills the wave alone (lane l takes samples l, l + 64, ...); smaller units are
 // packed side by side into power-of-two lane segments, so the lanes of a
 // wave stay busy when sample counts are small (adaptive pilots, uneven
 // counts).  Each unit's colour is the same canonical sum either way.
 //
-// Packet variants: six waves per SIMD (at most 80 VGPRs).  Traversal is
-// latency-bound, so resident waves set the throughput.  Left free, the
-// compiler takes 120-138 VGPRs (three or four waves); under the bound it moves
-// unit bookkeeping to scratch and reloads it outside the traversal loop.  The
-// per-ray variant's LDS stack columns allow few resident blocks anyway; four
-// waves (128 VGPRs) keep its traversal loop free of scratch.
-// kOnePass: every unit has at most 64 samples (a uniform count), so a round's
-// lanes trace once; the sums then need no registers across the traversal.
+// The workgroup dispatcher is the work queue: a grid has a wave per grab.  A
+// persistent grid with atomic counters per XCD spent 0.6 of its 0.70 ms on
+// those counters when 12,461 small units were rendered (all waves look
+// through all slices before they exit).
+//
+// Packet variants: six waves per SIMD (at most 80 VGPRs); five and four are
+// 4 and 13 % slower on the bee eye's batch.  The per-ray variant's LDS stack
+// columns allow few resident blocks anyway; four waves (128 VGPRs) keep its
+// traversal loop free of scratch.
+//
+// What a round needs after the walk is read anew from the kernel arguments
+// (fresh_args): held in scalar registers across it, the arguments spill.
+//
+// kOnePass: every unit has the same count of at most 64 samples, so a round's
+// lanes trace once, the sums need no registers across the traversal, and the
+// segments need no packing.
+// Packet workgroups are one wave: waves of uneven work then leave no slot idle
+// until their workgroup's last one ends (against four waves: bee eye's batch
+// 17.8 -> 16.0 ms, uneven batch 71.1 -> 63.6).
+constexpr int unit_threads(int traversal) { return traversal == kUnitPerRay ? kTraceThreads : 64; }
+
+struct RenderArgs {
+  SceneView S;
+  UnitLaunch U;
+  uint32_t omm_magic;   // floor(2^32 / omm_count), at most 2^32 - 1
+  uint32_t blocks;      // workgroups of work; the grid strides over them
+  uint32_t run;         // consecutive ones on one XCD
+};
+typedef __attribute__((address_space(4))) const RenderArgs KernelArgs;
+
+__device__ __forceinline__ KernelArgs* fresh_args() {
+  KernelArgs* p = (KernelArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
+// Pose and place in the processing order of unit u: u / omm_count by the
+// magic reciprocal, whose estimate is exact or one too small.
+__device__ __forceinline__ void split_unit(uint32_t u, uint32_t n, uint32_t magic, uint32_t* p, uint32_t* k) {
+  uint32_t q = __umulhi(u, magic);
+  uint32_t rest = u - q * n;
+  if (rest >= n) {
+    ++q;
+    rest -= n;
+  }
+  *p = q;
+  *k = rest;
+}
+
 template <bool kStats, bool kSamples, int kTrav, bool kOnePass = false>
-__global__ __launch_bounds__(kTraceThreads, kTrav == kUnitPerRay ? 4 : 6) void k_render_units(SceneView S,
-                                                                                             UnitLaunch U) {
-  // LDS (per-ray traversal only): one stack column per lane, laid out
-  // [depth][blockDim.x]; packets keep their stack in VGPR lanes
+__global__ __launch_bounds__(unit_threads(kTrav), kTrav == kUnitPerRay ? 4 : 6) void k_render_units(RenderArgs A) {
+  // LDS: per-ray traversal a stack column per lane, laid out
+  // [depth][blockDim.x]; wide packets a stack per wave
   extern __shared__ uint32_t unit_lds[];
   const int lane = threadIdx.x & 63;
   uint32_t* lane_stack = unit_lds + threadIdx.x;
-  const uint64_t units = (uint64_t)U.pose_count * (uint64_t)U.omm_count;
-  // The queue is split into kXcds slices of consecutive units with a counter
-  // each.  A wave takes units from its workgroup's XCD slice (neighbouring
-  // directions of the same poses share that XCD's L2) and, once the slice is
-  // empty, from the following slices; it exits when all are empty.
-  const uint64_t slice = (units + kXcds - 1) / kXcds;
-  uint32_t x = blockIdx.x % kXcds;
-  uint32_t tried = 0;
-  uint32_t w_steps = 0, w_tris = 0;   // packet node visits and leaf triangles of this wave
-  for (;;) {
-    uint64_t base = 0, s_end = 0;
-    while (tried < kXcds) {
-      const uint64_t s0 = (uint64_t)x * slice, s1 = min(units, s0 + slice);
-      uint32_t off = 0xffffffffu;
-      if (lane == 0 && s0 < s1) off = atomicAdd(U.queue + x, (uint32_t)U.units_per_grab);
-      off = (uint32_t)__builtin_amdgcn_readfirstlane((int)__shfl(off, 0));
-      if (s0 < s1 && s0 + off < s1) {
-        base = s0 + off;
-        s_end = s1;
-        break;
-      }
-      x = (x + 1u) % kXcds;
-      ++tried;
-    }
-    if (tried >= kXcds) {
-      if (U.packet_counts && lane == 0 && w_steps != 0u) {
-        atomicAdd(U.packet_counts, (unsigned long long)w_steps);
-        atomicAdd(U.packet_counts + 1, (unsigned long long)w_tris);
-      }
-      break;
-    }
-    const int G = (int)min((uint64_t)U.units_per_grab, s_end - base);
-    // lane g < G holds the sample count of unit base + g
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t units = (uint32_t)((uint64_t)A.U.pose_count * (uint64_t)A.U.omm_count);
+  uint32_t w_steps = 0, w_tris = 0;   // packet node fetches and leaf triangles of this wave
+  for (uint32_t b = blockIdx.x; b < fresh_args()->blocks; b += gridDim.x) {
+    const uint32_t G0 = (uint32_t)fresh_args()->U.units_per_grab;
+    const uint64_t first = (uint64_t)(xcd_run_block(b, fresh_args()->blocks, fresh_args()->run) *
+                                          (unit_threads(kTrav) / 64) + wave) * G0;
+    if (first >= units) continue;   // whole wave
+    const uint32_t base = (uint32_t)first;
+    const int G = (int)min(G0, units - base);
+    // lane g < G holds the sample count of a unit; rounds take the grab's
+    // units largest first, so that power-of-two segments tile the 64 lanes
+    // without gaps.  Sorted position q holds unit offset order[q] (units above
+    // 32 samples, which fill whole rounds, compare equal).
     uint32_t my_n = 0;
-    if (lane < G) {
-      int p, i;
-      uint32_t out;
-      locate_unit32(U, (uint32_t)base + (uint32_t)lane, &p, &i, &out);
-      my_n = unit_count(U, out, i);
+    int order = lane;
+    if (!kOnePass) {
+      KernelArgs* K = fresh_args();
+      if (lane < G) {
+        uint32_t p, k;
+        split_unit(base + (uint32_t)lane, (uint32_t)K->U.omm_count, K->omm_magic, &p, &k);
+        const uint32_t i = K->U.order ? K->U.order[k] : k;
+        my_n = K->U.unit_counts ? K->U.unit_counts[p * (uint32_t)K->U.omm_count + i]
+                                : K->U.omm_counts ? K->U.omm_counts[i] : (uint32_t)K->U.spp;
+      }
+      const uint32_t key = wave_sort_desc(lane < G ? ((min(my_n, 64u) + 1u) << 6) | (uint32_t)lane : 0u);
+      order = (int)(key & 63u);
+      my_n = (uint32_t)__shfl((int)my_n, order);
     }
-    // Rounds take the grab's units largest first: power-of-two segments in
-    // decreasing size tile the 64 lanes without gaps.  Sorted position q
-    // holds unit offset order[q] (units above 32 samples, which fill whole
-    // rounds, compare equal).  Output positions stay per unit.
-    const uint32_t key = wave_sort_desc(lane < G ? ((min(my_n, 64u) + 1u) << 6) | (uint32_t)lane : 0u);
-    const int order = (int)(key & 63u);
-    my_n = (uint32_t)__shfl((int)my_n, order);
     int g = 0;
     while (g < G) {
       // ---- build a round: which unit (slot) each lane serves ----
       int slot = -1, seg_off = 0, seg = 64;
       int g_end = g + 1;
-      const uint32_t n_first = (uint32_t)__builtin_amdgcn_readlane((int)my_n, g);
-      if (n_first > 32u) {
-        slot = g;
+      uint32_t n;
+      if (kOnePass) {
+        n = (uint32_t)fresh_args()->U.spp;
+        const int log_seg = n <= 1u ? 0 : 32 - __builtin_clz(n - 1u);
+        seg = 1 << log_seg;
+        slot = g + (lane >> log_seg);
+        seg_off = lane & ~(seg - 1);
+        g_end = min(G, g + (64 >> log_seg));
+        if (slot >= G) slot = -1;
       } else {
-        int cursor = 0;
-        g_end = g;
-        while (g_end < G) {
-          const uint32_t nj = (uint32_t)__builtin_amdgcn_readlane((int)my_n, g_end);
-          if (nj > 32u) break;
-          const int sj = pow2_at_least(nj);
-          const int a = (cursor + sj - 1) & ~(sj - 1);
-          if (a + sj > 64) break;
-          if (lane >= a && lane < a + sj) {
-            slot = g_end;
-            seg_off = a;
-            seg = sj;
+        const uint32_t n_first = (uint32_t)__builtin_amdgcn_readlane((int)my_n, g);
+        if (n_first > 32u) {
+          slot = g;
+        } else {
+          int cursor = 0;
+          g_end = g;
+          while (g_end < G) {
+            const uint32_t nj = (uint32_t)__builtin_amdgcn_readlane((int)my_n, g_end);
+            if (nj > 32u) break;
+            const int sj = pow2_at_least(nj);
+            const int a = (cursor + sj - 1) & ~(sj - 1);
+            if (a + sj > 64) break;
+            if (lane >= a && lane < a + sj) {
+              slot = g_end;
+              seg_off = a;
+              seg = sj;
+            }
+            cursor = a + sj;
+            ++g_end;
           }
-          cursor = a + sj;
-          ++g_end;
         }
+        n = (uint32_t)__shfl((int)my_n, slot < 0 ? 0 : slot);   // every lane takes part
       }
       // ---- this lane's unit ----
-      const int src = slot < 0 ? 0 : slot;
-      const int unit_off = __shfl(order, src);
-      int p, i;
+      const int unit_off = kOnePass ? max(slot, 0) : __shfl(order, slot < 0 ? 0 : slot);
+      if (slot < 0) n = 0u;
+      uint32_t p, i;
       {
-        uint32_t out_unused;
-        locate_unit32(U, (uint32_t)base + (uint32_t)unit_off, &p, &i, &out_unused);
+        KernelArgs* K = fresh_args();
+        split_unit(base + (uint32_t)unit_off, (uint32_t)K->U.omm_count, K->omm_magic, &p, &i);
+        if (K->U.order) i = K->U.order[i];
       }
-      const uint32_t n_src = (uint32_t)__shfl((int)my_n, src);  // every lane takes part in the shuffle
-      const uint32_t n = slot < 0 ? 0u : n_src;
-      const float inv = 1.0f / (float)(n > 0u ? n : 1u);
       // The lane's place in the round, the one register of round bookkeeping
-      // kept across the traversal (the rest is recomputed after it, which
-      // keeps the six-wave kernel's unit state out of scratch): bit 16 set
-      // when the lane serves a unit, bits 8-10 log2 of its segment, bits 0-6
-      // the lane's first sample in its unit (lane - segment start).
+      // kept across the traversal: bit 16 set when the lane serves a unit,
+      // bits 8-10 log2 of its segment, bits 0-6 the lane's first sample in
+      // its unit (lane - segment start).
       const uint32_t desc = (slot >= 0 ? 0x10000u : 0u) | ((uint32_t)__builtin_ctz((unsigned)seg) << 8) |
                             (uint32_t)(lane - seg_off);
-      float r = 0.0f, gg = 0.0f, b = 0.0f;
+      float r = 0.0f, gg = 0.0f, bl = 0.0f;
       float sr = 0.0f, sg = 0.0f, sb = 0.0f, sd = 0.0f, sd2 = 0.0f, sh = 0.0f;
       for (uint32_t c0 = 0; __ballot(c0 + (desc & 127u) < n) != 0ull; c0 += 64u) {
-        const uint32_t s = c0 + (desc & 127u);
-        const bool active = s < n;
+        const bool active = c0 + (desc & 127u) < n;
         Ray ray;
         if (active) {
-          const U4 rnd = sample_randoms(U.seed, U.eye, (uint32_t)i, U.sample_base + s, U.frame,
-                                        U.pose_base + (uint32_t)p);
-          ray = generate_ray(U.omms[i], U.poses[p], rnd);
+          KernelArgs* K = fresh_args();
+          const U4 rnd = sample_randoms(K->U.seed, K->U.eye, i, K->U.sample_base + c0 + (desc & 127u), K->U.frame,
+                                        K->U.pose_base + p);
+          ray = generate_ray(K->U.omms[i], K->U.poses[p], rnd);
         } else {
           ray.ox = ray.oy = ray.oz = 0.0f;
           ray.dx = ray.dy = 0.0f;
@@ -632,24 +668,36 @@ __global__ __launch_bounds__(kTraceThreads, kTrav == kUnitPerRay ? 4 : 6) void k
           ray.tmin = 0.0f;
           ray.tmax = 1.0f;
         }
-        const RayPre rp = precompute_ray(ray);
         Hit h;
-        if (kTrav == kUnitPerRay) {
-          h.t = rp.tmax;
-          h.k = h.id = 0xffffffffu;
-          h.b1 = h.b2 = 0.0f;
-          if (active) closest_hit(S, rp, lane_stack, (int)blockDim.x, h);
-        } else {
-          packet_hits<kTrav>(S, ray, rp, active, unit_lds, h, w_steps, w_tris);
+        {
+          KernelArgs* K = fresh_args();
+          SceneView S;
+          S.nodes = K->S.nodes;
+          S.tris = K->S.tris;
+          S.wide = WideTree{K->S.wide.nodes, K->S.wide.tris, K->S.wide.root, K->S.wide.stack, K->S.wide.spread,
+                            K->S.wide.range};
+          S.node_count = K->S.node_count;
+          S.fault = K->S.fault;
+          const RayPre rp = precompute_ray(ray);
+          if (kTrav == kUnitPerRay) {
+            h.t = rp.tmax;
+            h.k = h.id = 0xffffffffu;
+            h.b1 = h.b2 = 0.0f;
+            if (active) closest_hit(S, rp, lane_stack, (int)blockDim.x, h);
+          } else {
+            packet_hits<kTrav>(S, ray, rp, active, unit_lds, h, w_steps, w_tris);
+          }
         }
         if (active) {
-          const V3 c = shade(S, h, ray.dx, ray.dy, ray.dz);
+          KernelArgs* K = fresh_args();
+          const V3 c = shade(K->S.cols, K->S.texels, K->S.textures, K->S.sky_mode, h, ray.dx, ray.dy, ray.dz);
+          const float inv = 1.0f / (float)n;
           r = r + c.x * inv;
           gg = gg + c.y * inv;
-          b = b + c.z * inv;
+          bl = bl + c.z * inv;
           const bool hit = h.id != 0xffffffffu;
           if (kSamples)
-            U.samples[U.sample_offsets[(uint32_t)p * (uint32_t)U.omm_count + (uint32_t)i] + s] =
+            K->U.samples[K->U.sample_offsets[p * (uint32_t)K->U.omm_count + i] + c0 + (desc & 127u)] =
                 make_float4(c.x, c.y, c.z, hit ? h.t : -1.0f);
           if (kStats) {
             sr += c.x * c.x;
@@ -666,7 +714,7 @@ __global__ __launch_bounds__(kTraceThreads, kTrav == kUnitPerRay ? 4 : 6) void k
       const int seg_len = 1 << ((desc >> 8) & 7u);
       r = segment_sum(r, seg_len);
       gg = segment_sum(gg, seg_len);
-      b = segment_sum(b, seg_len);
+      bl = segment_sum(bl, seg_len);
       if (kStats) {
         sr = segment_sum(sr, seg_len);
         sg = segment_sum(sg, seg_len);
@@ -676,37 +724,28 @@ __global__ __launch_bounds__(kTraceThreads, kTrav == kUnitPerRay ? 4 : 6) void k
         sh = segment_sum(sh, seg_len);
       }
       if ((desc & 0x1007fu) == 0x10000u) {   // the first lane of a unit's segment
-        const uint32_t out = (uint32_t)p * (uint32_t)U.omm_count + (uint32_t)i;
-        U.colours[out] = make_float4(r, gg, b, (float)n);
+        KernelArgs* K = fresh_args();
+        const uint32_t out = p * (uint32_t)K->U.omm_count + i;
+        K->U.colours[out] = make_float4(r, gg, bl, (float)n);
         if (kStats) {
           // E[c^2] - E[c]^2 with E[c] the unit's mean colour
+          const float inv = 1.0f / (float)(n > 0u ? n : 1u);
           const float vr = fmaxf(sr * inv - r * r, 0.0f);
           const float vg = fmaxf(sg * inv - gg * gg, 0.0f);
-          const float vb = fmaxf(sb * inv - b * b, 0.0f);
+          const float vb = fmaxf(sb * inv - bl * bl, 0.0f);
           const float md = sd * inv;
-          U.stats[2 * (size_t)out] = make_float4(vr, vg, vb, sh * inv);
-          U.stats[2 * (size_t)out + 1] = make_float4(md, fmaxf(sd2 * inv - md * md, 0.0f), 0.0f, 0.0f);
+          K->U.stats[2 * (size_t)out] = make_float4(vr, vg, vb, sh * inv);
+          K->U.stats[2 * (size_t)out + 1] = make_float4(md, fmaxf(sd2 * inv - md * md, 0.0f), 0.0f, 0.0f);
         }
       }
       g = g_end;
     }
   }
-}
-
-// Workgroups are handed to the 8 XCDs round-robin (block b to XCD b % 8),
-// and each XCD has its own L2.  Logical blocks are therefore dealt to XCDs in
-// runs of kXcdRun consecutive blocks: the queue is in Morton order of the
-// ommatidial axes, so an XCD's resident waves look in neighbouring directions
-// and share BVH nodes in its L2, while runs still alternate between XCDs so
-// that each gets its share of costly directions.  The mapping is a
-// bijection, so results do not depend on it.
-constexpr uint32_t kXcdRun = 16;
-
-__device__ __forceinline__ uint32_t xcd_logical_block(uint32_t b, uint32_t blocks) {
-  const uint32_t span = kXcds * kXcdRun;
-  if (b >= (blocks / span) * span) return b;
-  const uint32_t x = b % kXcds, j = b / kXcds;
-  return ((j / kXcdRun) * kXcds + x) * kXcdRun + j % kXcdRun;
+  unsigned long long* counts = fresh_args()->U.packet_counts;
+  if (counts && lane == 0 && w_steps != 0u) {
+    atomicAdd(counts, (unsigned long long)w_steps);
+    atomicAdd(counts + 1, (unsigned long long)w_tris);
+  }
 }
 
 // Split launch of units with a uniform sample count n, per-ray traversal:
@@ -1212,29 +1251,25 @@ static int g_trace_mode = kTracePacketWide;
 static const char* g_last_kernel = "";
 static bool g_split = true;
 
+using UnitsKernel = void (*)(RenderArgs);
+
+// A uniform count of at most 64 samples per unit (the adaptive pilot, uniform
+// batches of few samples): every round traces once.
+static bool one_pass(const UnitLaunch& U) { return !U.omm_counts && !U.unit_counts && U.spp <= 64; }
+
 template <int kTrav>
-static void launch_units_variant(const UnitLaunch& U, const SceneView& v, int blocks, size_t lds,
-                                 hipStream_t stream) {
-  const dim3 grid(blocks), block(kTraceThreads);
-  // a uniform count of at most 64 samples per unit (the adaptive pilot, uniform
-  // batches of few samples): every round traces once
-  const bool one = !U.omm_counts && !U.unit_counts && U.spp <= 64;
-  if (U.stats && U.samples && one)
-    hipLaunchKernelGGL((k_render_units<true, true, kTrav, true>), grid, block, lds, stream, v, U);
-  else if (U.stats && one)
-    hipLaunchKernelGGL((k_render_units<true, false, kTrav, true>), grid, block, lds, stream, v, U);
-  else if (U.samples && one)
-    hipLaunchKernelGGL((k_render_units<false, true, kTrav, true>), grid, block, lds, stream, v, U);
-  else if (one)
-    hipLaunchKernelGGL((k_render_units<false, false, kTrav, true>), grid, block, lds, stream, v, U);
-  else if (U.stats && U.samples)
-    hipLaunchKernelGGL((k_render_units<true, true, kTrav>), grid, block, lds, stream, v, U);
-  else if (U.stats)
-    hipLaunchKernelGGL((k_render_units<true, false, kTrav>), grid, block, lds, stream, v, U);
-  else if (U.samples)
-    hipLaunchKernelGGL((k_render_units<false, true, kTrav>), grid, block, lds, stream, v, U);
-  else
-    hipLaunchKernelGGL((k_render_units<false, false, kTrav>), grid, block, lds, stream, v, U);
+static UnitsKernel units_kernel_variant(const UnitLaunch& U) {
+  const bool one = one_pass(U);
+  if (U.stats && U.samples) return one ? k_render_units<true, true, kTrav, true> : k_render_units<true, true, kTrav>;
+  if (U.stats) return one ? k_render_units<true, false, kTrav, true> : k_render_units<true, false, kTrav>;
+  if (U.samples) return one ? k_render_units<false, true, kTrav, true> : k_render_units<false, true, kTrav>;
+  return one ? k_render_units<false, false, kTrav, true> : k_render_units<false, false, kTrav>;
+}
+
+static UnitsKernel units_kernel_of(const UnitLaunch& U) {
+  if (U.traversal == kUnitPerRay) return units_kernel_variant<kUnitPerRay>(U);
+  if (U.traversal == kUnitPacketWide) return units_kernel_variant<kUnitPacketWide>(U);
+  return units_kernel_variant<kUnitPacket>(U);
 }
 
 static void launch_chunks(const UnitLaunch& U, const SceneView& v, int blocks, size_t lds, int chunks,
@@ -1248,19 +1283,6 @@ static void launch_chunks(const UnitLaunch& U, const SceneView& v, int blocks, s
     hipLaunchKernelGGL((k_render_chunks<false, true>), grid, block, lds, stream, v, U, chunks);
   else
     hipLaunchKernelGGL((k_render_chunks<false, false>), grid, block, lds, stream, v, U, chunks);
-}
-
-template <int kTrav>
-static const void* units_kernel_variant(const UnitLaunch& U) {
-  const bool one = !U.omm_counts && !U.unit_counts && U.spp <= 64;
-  if (U.stats && U.samples && one) return reinterpret_cast<const void*>(&k_render_units<true, true, kTrav, true>);
-  if (U.stats && one) return reinterpret_cast<const void*>(&k_render_units<true, false, kTrav, true>);
-  if (U.samples && one) return reinterpret_cast<const void*>(&k_render_units<false, true, kTrav, true>);
-  if (one) return reinterpret_cast<const void*>(&k_render_units<false, false, kTrav, true>);
-  if (U.stats && U.samples) return reinterpret_cast<const void*>(&k_render_units<true, true, kTrav>);
-  if (U.stats) return reinterpret_cast<const void*>(&k_render_units<true, false, kTrav>);
-  if (U.samples) return reinterpret_cast<const void*>(&k_render_units<false, true, kTrav>);
-  return reinterpret_cast<const void*>(&k_render_units<false, false, kTrav>);
 }
 
 static int device_cus() {
@@ -1291,33 +1313,27 @@ static int effective_traversal(const DeviceScene& scene, int traversal) {
   return traversal != kUnitPerRay && scene.stack_bound > kPacketStackMax ? (int)kUnitPerRay : traversal;
 }
 
-static const void* units_kernel_of(const UnitLaunch& U) {
-  if (U.traversal == kUnitPerRay) return units_kernel_variant<kUnitPerRay>(U);
-  if (U.traversal == kUnitPacketWide) return units_kernel_variant<kUnitPacketWide>(U);
-  return units_kernel_variant<kUnitPacket>(U);
-}
-
 int render_units_capacity(const DeviceScene& scene, const UnitLaunch& U_in) {
   UnitLaunch U = U_in;
   U.traversal = effective_traversal(scene, U.traversal);
-  const void* fn = units_kernel_of(U);
+  const int threads = unit_threads(U.traversal);
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kTraceThreads, units_lds_bytes(scene, U.traversal)) !=
-          hipSuccess ||
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(units_kernel_of(U)), threads,
+                                                   units_lds_bytes(scene, U.traversal, threads / 64)) != hipSuccess ||
       per_cu <= 0)
-    per_cu = 4;
-  return device_cus() * per_cu;
+    per_cu = 4 * kTraceThreads / threads;
+  return std::max(1, device_cus() * per_cu * threads / kTraceThreads);
 }
 
 bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipStream_t stream, std::string* err) {
   UnitLaunch U = U_in;
   const uint64_t units = (uint64_t)U.pose_count * (uint64_t)U.omm_count;
   if (units == 0) return true;
-  if (units > 0xffffffffull - 65536ull) {
+  if (units > kMaxLaunchUnits) {
     if (err) *err = "render_units: too many units for one launch";
     return false;
   }
-  if (!U.queue || !U.colours || (U.samples && !U.sample_offsets)) {
+  if (!U.colours || (U.samples && !U.sample_offsets)) {
     if (err) *err = "render_units: incomplete launch description";
     return false;
   }
@@ -1332,7 +1348,6 @@ bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipSt
     return false;
   }
   const int capacity = render_units_capacity(scene, U);
-  int blocks = U.blocks > 0 ? U.blocks : capacity;
   const SceneView v = view_of(scene);
   // Split launch: uniform counts and fewer units than two per wave slot of
   // the device (a single pose, typically), when the caller gave scratch: each
@@ -1404,23 +1419,30 @@ bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipSt
     g_last_kernel = "k_render_chunks";
     return check_launch("render_chunks", err);
   }
-  // units per queue grab: as given, or (0) as many as keep two grabs per
-  // resident wave, at most auto_grab_max
-  UnitLaunch G = U;
-  if (G.units_per_grab <= 0)
-    G.units_per_grab = (int)std::min<uint64_t>((uint64_t)std::max(G.auto_grab_max, 1),
-                                               std::max<uint64_t>(1, units / (2 * resident_waves)));
-  G.units_per_grab = std::min(G.units_per_grab, kMaxUnitsPerGrab);
-  const uint64_t need = (units + (uint64_t)G.units_per_grab - 1) / (uint64_t)G.units_per_grab;
-  const uint64_t waves = (uint64_t)blocks * (kTraceThreads / 64);
-  if (waves > need) blocks = (int)((need + (kTraceThreads / 64) - 1) / (kTraceThreads / 64));
-  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, stream, G.queue, (uint32_t)kQueueWords, 0u);
-  if (G.traversal == kUnitPerRay)
-    launch_units_variant<kUnitPerRay>(G, v, blocks, lds, stream);
-  else if (G.traversal == kUnitPacketWide)
-    launch_units_variant<kUnitPacketWide>(G, v, blocks, lds, stream);
-  else
-    launch_units_variant<kUnitPacket>(G, v, blocks, lds, stream);
+  // Units per wave: as given, or (0) as many as leave four waves for every
+  // resident slot, at most auto_grab_max, but enough to fill a wave's lanes.
+  RenderArgs A{v, U, 0, 0, 1};
+  if (A.U.units_per_grab <= 0) {
+    uint64_t fill = 1;
+    if (one_pass(U))
+      for (uint64_t seg = 64; seg > 1 && seg / 2 >= (uint64_t)std::max(U.spp, 1); seg /= 2) fill *= 2;
+    A.U.units_per_grab = (int)std::max<uint64_t>(
+        fill, std::min<uint64_t>((uint64_t)std::max(U.auto_grab_max, 1), units / (4 * resident_waves)));
+  }
+  A.U.units_per_grab = std::min(A.U.units_per_grab, kMaxUnitsPerGrab);
+  A.omm_magic = (uint32_t)std::min<uint64_t>(0xffffffffull, (1ull << 32) / (uint64_t)U.omm_count);
+  const int threads = unit_threads(U.traversal);
+  const uint64_t per_block = (uint64_t)A.U.units_per_grab * (uint64_t)(threads / 64);
+  A.blocks = (uint32_t)((units + per_block - 1) / per_block);
+  // eight runs of consecutive workgroups per XCD: long enough for its L2 to
+  // hold a pose's surroundings, short enough to even out the XCDs' work (4 to
+  // 16 runs within 1 %, 64 runs 3-10 % slower)
+  A.run = std::max<uint32_t>(1u, A.blocks / (kXcds * 8u));
+  const uint32_t grid =
+      U.blocks > 0 ? (uint32_t)std::min<uint64_t>((uint64_t)U.blocks * (uint64_t)(kTraceThreads / threads), A.blocks)
+                   : A.blocks;
+  hipLaunchKernelGGL(units_kernel_of(U), dim3(grid), dim3(threads), units_lds_bytes(scene, U.traversal, threads / 64),
+                     stream, A);
   g_last_kernel = "k_render_units";
   return check_launch("render_units", err);
 }

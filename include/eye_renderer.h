@@ -178,11 +178,9 @@ double renderPoseBatch(const float* poses, size_t poseCount, float* rgbOut);
  * (r, g, b, samples) (16-byte aligned).  The same units, random streams and
  * colours as renderPoseBatch at the same poses.  The work is enqueued on
  * `stream` (a hipStream_t; NULL: the library's stream) and not waited for.
- * The unit renderer's work counters live in a fixed 256-byte device array
- * (one per GPU, held until the process ends, cleared by a kernel at the start
- * of every call); nothing is allocated and no hipMalloc/hipFree is called.
- * Calls that overlap on one GPU race on that array.  Limits: at most
- * 2^32 - 65537 (pose, ommatidium) units per call; the current eye must be
+ * Nothing is allocated, no hipMalloc/hipFree is called and no scratch is
+ * used: calls may overlap on several streams.  Limits: at most 2^32 - 65537
+ * (pose, ommatidium) units per call; the current eye must be
  * resident, i.e. rendered by renderFrame or renderPoseBatch since its
  * ommatidia or sample counts last changed (those calls upload it and may
  * allocate).  A packet traversal fault is reported by the next call that
@@ -300,11 +298,11 @@ void setTaskSplit(int mode);
  * (0 when the split was off for that render or nothing was long enough).  No counterpart
  * in the reference (diagnostic of this renderer's scheduling). */
 int getCurrentEyeTaskSplits(void);
-/* Launch shape of the persistent unit renderer: ommatidia taken from the work
- * queue per grab (0 = automatic, at most 64: a wave holds one grab's sample
- * counts in its lanes), and blocks of 256 threads (0 = every resident slot
- * once).  The adaptive passes keep the blocks and traversal but choose their
- * own grab size. */
+/* Launch shape of the unit renderer: ommatidia that a wave renders one after
+ * another (0 = automatic, at most 64: a wave holds their sample counts in its
+ * lanes), and blocks of 256 threads, which stride over the work (0 = a wave
+ * per grab of ommatidia).  The adaptive passes keep the blocks and traversal
+ * but choose their own grab size. */
 void setRenderTuning(int unitsPerGrab, int blocks);
 /* Writes the current launch shape: units per grab, blocks, traversal mode. */
 int getRenderTuning(int* shape3);

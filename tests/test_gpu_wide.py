@@ -157,3 +157,35 @@ def test_rays_that_hit_nothing(lib, tmp_path):
     omm = eye_of(axes, -2.0 * axes, 0.1)
     for split in (True, False):
         check(lib, tmp_path, pos, col, omm, 9, split=split, modes=(2,))
+
+
+@pytest.mark.parametrize("grab,blocks", [(0, 0), (1, 1), (5, 3), (64, 1), (7, 100000)])
+@pytest.mark.parametrize("counts", [None, "uneven"])
+def test_unit_grid_shapes(lib, tmp_path, grab, blocks, counts):
+    """Any grab size and grid, down to one workgroup that strides over all the
+    work, gives every (pose, ommatidium) unit once: batches of an ommatidium
+    count that is not a power of two, at one and at several poses."""
+    pos, col = soup(800, 15)
+    omm = eye_of(random_axes(131, 9), -2.0 * random_axes(131, 9), 0.1)
+    sc = scenes.Scene([scenes.Mesh("m", pos, np.arange(len(pos), dtype=np.uint32).reshape(-1, 3), col)],
+                      eyes=[scenes.Eye("eye", omm)])
+    lib.loadGlTFscene(str(scenes.write_gltf(tmp_path, "s", sc)).encode())
+    er.gotoFirstCompoundEye(lib)
+    er.set_ommatidia_np(lib, omm)
+    n = None if counts is None else scenes.log_uniform_counts(131, 1, 130, seed=4)
+    lib.setCurrentEyeSamplesPerOmmatidium(13)
+    er.set_sample_counts(lib, n)
+    poses6 = np.zeros((5, 6), np.float32)
+    poses6[:, 0] = np.linspace(-0.2, 0.2, 5)
+    poses6[:, 4] = np.arange(5)
+    poses12 = np.stack([oracle.pose12(p) for p in poses6])
+    lib.setRenderTuning(grab, blocks)
+    try:
+        for k in (1, 5):
+            want = oracle.OracleScene.from_scene(sc).render(omm, poses12[:k], spp=13, counts=n,
+                                                            frame=lib.getCurrentEyeFrameIndex())
+            _, rgb = er.render_batch_np(lib, poses6[:k])
+            assert np.array_equal(rgb, want["colour_gpu_order"]), k
+    finally:
+        lib.setRenderTuning(0, 0)
+        er.set_sample_counts(lib, None)
