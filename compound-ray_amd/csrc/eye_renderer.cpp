@@ -59,18 +59,16 @@ struct EyeState {
   size_t d_colours_cap = 0;
   bool has_render = false;
   uint64_t rendered_rays = 0;
-  // scratch of split renders (per-lane chunk values, per-unit counters)
-  float4* d_chunk_partial = nullptr;
+  // scratch of split renders (per-lane chunk values)
+  float* d_chunk_partial = nullptr;
   size_t d_chunk_partial_cap = 0;
-  uint32_t* d_chunk_done = nullptr;
-  size_t d_chunk_done_cap = 0;
   // long-task split of split renders: per task the packet steps of the last
   // render and a flag, the split list and counters (render.h, UnitLaunch)
   uint32_t* d_split = nullptr;
   size_t d_split_cap = 0;
   uint64_t split_tasks = 0;       // tasks the buffers are laid out for
   bool split_valid = false;       // the cost words hold the steps of a render of those tasks
-  uint32_t split_listed[3] = {0, 0, 0};   // tasks the last render listed per tier
+  const uint32_t* split_counts = nullptr;   // device: tasks the last render listed per tier (null: none)
   uint64_t split_generation = 0;  // scene the costs were measured on
   // automatic choice: renders of the same tasks since the last trial began,
   // and the shortest trace time (ms) of the trial's renders without / with
@@ -248,7 +246,6 @@ void free_scene() {
     if (e.d_colours) (void)hipFree(e.d_colours);
     if (e.d_proj_ids) (void)hipFree(e.d_proj_ids);
     if (e.d_chunk_partial) (void)hipFree(e.d_chunk_partial);
-    if (e.d_chunk_done) (void)hipFree(e.d_chunk_done);
     if (e.d_split) (void)hipFree(e.d_split);
     if (e.d_counts) (void)hipFree(e.d_counts);
     if (e.d_sample_offsets) (void)hipFree(e.d_sample_offsets);
@@ -274,6 +271,7 @@ constexpr uint32_t kSplitTrialEvery = 1000;
 
 void split_restart(EyeState& e) {
   e.split_valid = false;
+  e.split_counts = nullptr;
   e.split_frames = 0;
   e.split_ms[0] = e.split_ms[1] = 1e30f;
 }
@@ -461,12 +459,20 @@ double render_compound(EyeState& e, const Cam& c) {
   if (record) ensure_device(&e.d_samples, &e.d_samples_cap, (size_t)total);
   ensure_device(&e.d_colours, &e.d_colours_cap, e.omms.size());
   ensure_frame_buffer();
-  hip_check(hipMemcpyAsync(s.d_pose, &c.pose, sizeof(Pose), hipMemcpyHostToDevice, s.stream), "upload pose");
-  EyeLaunch L = launch_of(e, s.d_pose, 1);
+  const int omm_count = (int)e.omms.size();
   std::string err;
   const auto t0 = std::chrono::steady_clock::now();
   hip_check(hipEventRecord(s.ev[0], s.stream), "event");
-  UnitLaunch U = unit_launch_of(e, s.d_pose, 1);
+  UnitLaunch U = unit_launch_of(e, nullptr, 1);
+  U.host_pose = &c.pose;
+  U.traced = s.ev[1];
+  bool frame_done = false;
+  if (e.shader != "single_dimension" && e.shader != "raw_ommatidial_samples" &&
+      e.shader.compare(0, 10, "spherical_") != 0) {
+    U.frame_pixels = s.d_frame;   // single_dimension_fast
+    U.frame_width = s.height > 0 ? s.width : 0;
+    U.frame_done = &frame_done;
+  }
   if (record) {
     U.samples = e.d_samples;
     U.sample_offsets = e.d_sample_offsets;
@@ -474,12 +480,9 @@ double render_compound(EyeState& e, const Cam& c) {
   if (e.counts.empty()) {
     // one pose: let the chunks of each ommatidium's samples spread over waves
     const size_t chunks = ((size_t)e.spp + 63) / 64;
-    ensure_device(&e.d_chunk_partial, &e.d_chunk_partial_cap, e.omms.size() * chunks * 64);
-    ensure_device(&e.d_chunk_done, &e.d_chunk_done_cap, e.omms.size());
+    ensure_device(&e.d_chunk_partial, &e.d_chunk_partial_cap, e.omms.size() * chunks * 192);
     U.chunk_partial = e.d_chunk_partial;
     U.chunk_partial_cap = e.d_chunk_partial_cap;
-    U.chunk_done = e.d_chunk_done;
-    U.chunk_done_cap = e.d_chunk_done_cap;
     // the packet task kernel's long-task split, planned from the last render
     const uint64_t tasks = (uint64_t)e.omms.size() * chunks;
     if (e.split_tasks != tasks || e.split_generation != s.scene.generation) {
@@ -500,7 +503,6 @@ double render_compound(EyeState& e, const Cam& c) {
       U.split_flag = U.split_cost + tasks;
       U.split_list = U.split_flag + tasks;
       U.split_count = U.split_list + kSplitListMax;
-      U.split_sub_done = U.split_count + kSplitCountWords;
       U.split_tasks = tasks;
       U.split_plan = plan;
     }
@@ -509,19 +511,15 @@ double render_compound(EyeState& e, const Cam& c) {
     split_restart(e);
     throw std::runtime_error(err);
   }
-  e.split_listed[0] = e.split_listed[1] = e.split_listed[2] = 0;
+  e.split_counts = nullptr;
   const bool tasks_kernel = std::strcmp(last_render_kernel(), "k_render_tasks") == 0;
   if (U.split_cost && tasks_kernel) {
-    if (U.split_plan)
-      hip_check(hipMemcpyAsync(e.split_listed, U.split_count, sizeof(e.split_listed), hipMemcpyDeviceToHost,
-                               s.stream),
-                "split count");
+    if (U.split_plan) e.split_counts = U.split_count;
     e.split_valid = true;
   } else {
     e.split_valid = false;
   }
   if (!tasks_kernel) split_restart(e);
-  hip_check(hipEventRecord(s.ev[1], s.stream), "event");
   hip_check(hipEventRecord(s.ev[2], s.stream), "event");
   bool ok = true;
   int sph = -1;
@@ -535,7 +533,7 @@ double render_compound(EyeState& e, const Cam& c) {
     const int pixels = s.width * s.height;
     if (e.proj_w != s.width || e.proj_h != s.height || e.proj_variant != sph || e.proj_version != e.omm_version) {
       ensure_device(&e.d_proj_ids, &e.d_proj_cap, (size_t)std::max(pixels, 1));
-      ok = launch_spherical_ids(e.d_omms, L.omm_count, s.width, s.height, sph, e.d_proj_ids, s.stream, &err);
+      ok = launch_spherical_ids(e.d_omms, omm_count, s.width, s.height, sph, e.d_proj_ids, s.stream, &err);
       e.proj_w = s.width;
       e.proj_h = s.height;
       e.proj_variant = sph;
@@ -543,12 +541,12 @@ double render_compound(EyeState& e, const Cam& c) {
     }
     if (ok) ok = launch_frame_lookup(e.d_colours, e.d_proj_ids, pixels, sph_ids, s.d_frame, s.stream, &err);
   } else if (e.shader == "single_dimension")
-    ok = launch_frame_single_dim(e.d_colours, L.omm_count, s.d_frame, s.width, s.height, s.stream, &err);
+    ok = launch_frame_single_dim(e.d_colours, omm_count, s.d_frame, s.width, s.height, s.stream, &err);
   else if (e.shader == "raw_ommatidial_samples")
-    ok = launch_frame_raw_samples(e.d_samples, e.counts.empty() ? nullptr : e.d_offsets, L.omm_count, e.spp,
+    ok = launch_frame_raw_samples(e.d_samples, e.counts.empty() ? nullptr : e.d_offsets, omm_count, e.spp,
                                   s.d_frame, s.width, s.height, s.stream, &err);
-  else
-    ok = launch_frame_single_dim_fast(e.d_colours, L.omm_count, s.d_frame, s.width, s.stream, &err);
+  else if (!frame_done && s.height > 0)
+    ok = launch_frame_single_dim_fast(e.d_colours, omm_count, s.d_frame, s.width, s.stream, &err);
   if (!ok) throw std::runtime_error(err);
   hip_check(hipEventRecord(s.ev[3], s.stream), "event");
   hip_check(hipStreamSynchronize(s.stream), "render");
@@ -1662,8 +1660,13 @@ void setTaskSplit(int mode) {
 }
 
 int getCurrentEyeTaskSplits(void) {
+  ABI_GUARD_BEGIN
   EyeState* e = current_eye();
-  return e ? (int)(e->split_listed[0] + e->split_listed[1]) : 0;
+  if (!e || !e->split_counts) return 0;
+  uint32_t listed[2] = {0, 0};   // read when asked for: a copy per frame would cost it 11 us
+  hip_check(hipMemcpy(listed, e->split_counts, sizeof(listed), hipMemcpyDeviceToHost), "split count");
+  return (int)(listed[0] + listed[1]);
+  ABI_GUARD_END(return 0)
 }
 
 void setRenderTuning(int unitsPerGrab, int blocks) {

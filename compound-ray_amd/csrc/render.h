@@ -36,16 +36,12 @@ constexpr int kSplit1Max = 2048;            // tier 2: tasks started early, whol
 constexpr uint32_t kSplitMinSteps = 128;    // tiers 0 and 1: a task of fewer packet steps is never split
 constexpr uint32_t kSplitEarlyMinSteps = 64;  // tier 2: nor started early
 constexpr int kSplitListMax = kSplit4Max + kSplit2Max + kSplit1Max;
-constexpr int kSplitSubMax = kSplit4Max + kSplit2Max;   // listed tasks traced as several packets
 constexpr int kSplitSubWaves = 4 * kSplit4Max + 2 * kSplit2Max + kSplit1Max;
 constexpr int kSplitCountWords = 8;         // listed per tier, then the tiers' thresholds in steps
 constexpr int kSplitBins = 256;             // threshold search: histogram bins of 8 steps
 // Device words of a split buffer for `tasks` tasks: cost and flag per task,
-// the tiers' lists, the counts and thresholds, a completion counter per
-// split task.
-constexpr uint64_t split_buffer_words(uint64_t tasks) {
-  return 2 * tasks + (uint64_t)kSplitListMax + kSplitCountWords + kSplitSubMax;
-}
+// the tiers' lists, the counts and thresholds.
+constexpr uint64_t split_buffer_words(uint64_t tasks) { return 2 * tasks + (uint64_t)kSplitListMax + kSplitCountWords; }
 
 // Ommatidium-unit renderer.  A unit is one ommatidium at one pose; a wave
 // renders `units_per_grab` consecutive units, traces a unit's samples 64 at a
@@ -69,27 +65,32 @@ struct UnitLaunch {
                                         //   (mean inverse depth, its variance, 0, 0)
   float4* samples = nullptr;            // nullable: per-sample (r, g, b, t or -1)
   const uint64_t* sample_offsets = nullptr;  // first sample record of each unit
-  // Optional scratch for split launches (uniform sample counts and few
-  // units): each unit's 64-sample chunks go to different waves; per-lane
-  // chunk values (1 float4, 3 with stats) and a completion counter per unit.
-  float4* chunk_partial = nullptr;
-  uint64_t chunk_partial_cap = 0;       // float4 elements
-  uint32_t* chunk_done = nullptr;
-  uint64_t chunk_done_cap = 0;          // counters
+  // One pose, when `poses` is null (host memory, copied into the launch).
+  const Pose* host_pose = nullptr;
+  // Optional scratch for split launches (one host_pose, a uniform sample count
+  // and few units): each unit's 64-sample chunks go to different waves, which
+  // keep 3 floats per lane for the sums.
+  float* chunk_partial = nullptr;
+  uint64_t chunk_partial_cap = 0;       // floats: 192 per chunk
+  // Optional, split launches only: the frame whose first row shows ommatidium
+  // x in pixel x < frame_width; *frame_done tells whether it was written.
+  uchar4* frame_pixels = nullptr;
+  int frame_width = 0;
+  bool* frame_done = nullptr;
+  // Optional: recorded after the tracing kernel.
+  hipEvent_t traced = nullptr;
   // Optional long-task split of the packet task kernel (an eye rendered frame
   // after frame, one pose, uniform counts).  The packet steps each task took
   // in the last launch (split_cost, per task) predict this launch's longest
   // tasks, which are listed (split_list, three tiers of kSplit4Max,
   // kSplit2Max and kSplit1Max entries) and flagged (split_flag: tier + 1) and
   // traced first, split into packets of rays of neighbouring elevation or
-  // whole.  Results do not depend on it.  split_count: kSplitCountWords;
-  // split_sub_done: kSplitSubMax.  split_plan: split_cost holds the steps of
-  // a launch of the same tasks.
+  // whole.  Results do not depend on it.  split_count: kSplitCountWords.
+  // split_plan: split_cost holds the steps of a launch of the same tasks.
   uint32_t* split_cost = nullptr;
   uint32_t* split_flag = nullptr;
   uint32_t* split_list = nullptr;
   uint32_t* split_count = nullptr;      // [0..2] tasks listed per tier, [3..5] the tiers' thresholds
-  uint32_t* split_sub_done = nullptr;
   uint64_t split_tasks = 0;
   bool split_plan = false;
   // launch shape (results do not depend on it)

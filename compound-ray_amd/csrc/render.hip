@@ -449,14 +449,6 @@ __device__ __forceinline__ float segment_sum(float v, int seg) {
   return v;
 }
 
-// Pose, ommatidium and output slot of unit u of the processing order.
-__device__ __forceinline__ void locate_unit(const UnitLaunch& U, uint64_t u, int* p, int* i, uint64_t* out) {
-  *p = (int)(u / (uint64_t)U.omm_count);
-  const int k = (int)(u - (uint64_t)*p * (uint64_t)U.omm_count);
-  *i = U.order ? (int)U.order[k] : k;
-  *out = (uint64_t)*p * (uint64_t)U.omm_count + (uint64_t)*i;
-}
-
 // Bitonic sort of one value per lane, largest first, across the 64 lanes.
 template <int K, int J>
 __device__ __forceinline__ uint32_t sort_step(uint32_t v, int lane) {
@@ -494,16 +486,11 @@ __device__ __forceinline__ int pow2_at_least(uint32_t n) {
 // and share BVH nodes in its L2, while runs still alternate between XCDs so
 // that each gets its share of costly directions.  The mapping is a
 // bijection, so results do not depend on it.
-constexpr uint32_t kXcdRun = 16;
-
 __device__ __forceinline__ uint32_t xcd_run_block(uint32_t b, uint32_t blocks, uint32_t run) {
   const uint32_t span = kXcds * run;
   if (b >= (blocks / span) * span) return b;
   const uint32_t x = b % kXcds, j = b / kXcds;
   return ((j / run) * kXcds + x) * run + j % run;
-}
-__device__ __forceinline__ uint32_t xcd_logical_block(uint32_t b, uint32_t blocks) {
-  return xcd_run_block(b, blocks, kXcdRun);
 }
 
 // Unit renderer.  A wave takes units_per_grab consecutive units of the
@@ -537,9 +524,13 @@ constexpr int unit_threads(int traversal) { return traversal == kUnitPerRay ? kT
 struct RenderArgs {
   SceneView S;
   UnitLaunch U;
+  Pose pose;            // the one pose when U.poses is null
   uint32_t omm_magic;   // floor(2^32 / omm_count), at most 2^32 - 1
   uint32_t blocks;      // workgroups of work; the grid strides over them
   uint32_t run;         // consecutive ones on one XCD
+  // split launches: chunks per unit and the reciprocal of split_unit, tasks, 1 / spp
+  uint32_t chunks, chunk_magic, tasks;
+  float inv;
 };
 typedef __attribute__((address_space(4))) const RenderArgs KernelArgs;
 
@@ -547,6 +538,30 @@ __device__ __forceinline__ KernelArgs* fresh_args() {
   KernelArgs* p = (KernelArgs*)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(p));
   return p;
+}
+
+__device__ __forceinline__ Pose pose_of(KernelArgs* K, uint32_t p) {
+  if (K->U.poses) return K->U.poses[p];
+  Pose P;
+  for (int a = 0; a < 3; ++a) {
+    P.pos[a] = K->pose.pos[a];
+    P.x[a] = K->pose.x[a];
+    P.y[a] = K->pose.y[a];
+    P.z[a] = K->pose.z[a];
+  }
+  return P;
+}
+
+// What a traversal needs of the scene.
+__device__ __forceinline__ SceneView walk_view(KernelArgs* K) {
+  SceneView S;
+  S.nodes = K->S.nodes;
+  S.tris = K->S.tris;
+  S.wide = WideTree{K->S.wide.nodes, K->S.wide.tris, K->S.wide.root, K->S.wide.stack, K->S.wide.spread,
+                    K->S.wide.range};
+  S.node_count = K->S.node_count;
+  S.fault = K->S.fault;
+  return S;
 }
 
 // Pose and place in the processing order of unit u: u / omm_count by the
@@ -660,7 +675,7 @@ __global__ __launch_bounds__(unit_threads(kTrav), kTrav == kUnitPerRay ? 4 : 6) 
           KernelArgs* K = fresh_args();
           const U4 rnd = sample_randoms(K->U.seed, K->U.eye, i, K->U.sample_base + c0 + (desc & 127u), K->U.frame,
                                         K->U.pose_base + p);
-          ray = generate_ray(K->U.omms[i], K->U.poses[p], rnd);
+          ray = generate_ray(K->U.omms[i], pose_of(K, p), rnd);
         } else {
           ray.ox = ray.oy = ray.oz = 0.0f;
           ray.dx = ray.dy = 0.0f;
@@ -671,13 +686,7 @@ __global__ __launch_bounds__(unit_threads(kTrav), kTrav == kUnitPerRay ? 4 : 6) 
         Hit h;
         {
           KernelArgs* K = fresh_args();
-          SceneView S;
-          S.nodes = K->S.nodes;
-          S.tris = K->S.tris;
-          S.wide = WideTree{K->S.wide.nodes, K->S.wide.tris, K->S.wide.root, K->S.wide.stack, K->S.wide.spread,
-                            K->S.wide.range};
-          S.node_count = K->S.node_count;
-          S.fault = K->S.fault;
+          const SceneView S = walk_view(K);
           const RayPre rp = precompute_ray(ray);
           if (kTrav == kUnitPerRay) {
             h.t = rp.tmax;
@@ -748,17 +757,23 @@ __global__ __launch_bounds__(unit_threads(kTrav), kTrav == kUnitPerRay ? 4 : 6) 
   }
 }
 
-// Split launch of units with a uniform sample count n, per-ray traversal:
-// task t is chunk t % C of queue position t / C (C = ceil(n / 64)), so that a
-// single pose's few units still fill the GPU.  Wave w of logical block L is
-// task 4L + w; there is no task loop.  Lane l of a task keeps the terms of
-// its one sample (scaled colour, and the statistics terms) in `partial`; the
-// wave that completes a unit's last chunk adds the chunks lane by lane in
-// chunk order and then across the wave, which gives the same sums as
-// k_render_units (there a lane adds samples l, l + 64, ... in this order).
+// Split launch of one pose's units with a uniform sample count n: task t is
+// chunk t % C of unit t / C of the processing order (C = ceil(n / 64)), so
+// that a single pose's few units still fill the GPU.  A wave traces one
+// task; lane l keeps the scaled colour of its one sample in `partial` (three
+// planes of 64 floats per task), and k_reduce_tasks adds a unit's chunks lane
+// by lane in chunk order and then across the wave, which gives the same sums
+// as k_render_units (there a lane adds samples l, l + 64, ... in this order).
 //
-// The rays of a task are traversed one per lane (an LDS stack column per
-// lane), so lanes past n simply skip the traversal.
+// Two kernels, because completing units inside the task kernel (a counter
+// per unit, behind a device-scope fence per task that writes back the XCD's
+// L2) cost more than the traversal: 1,000 ommatidia x 3,200 samples 1.19 ms
+// in the task kernel against 0.17 and 0.012 in the two, 1 sample 53 against
+// 23 us.
+//
+// A unit of one chunk needs no partial sums: its wave writes the colour.  Where
+// the frame shows ommatidium x in pixel x of its first row, the wave that
+// knows a colour writes its pixel too (`frame`, `frame_width`).
 //
 // Why no persistent task loop: a loop whose body takes its task from a lane-0
 // atomic broadcast with __shfl and ends in lane-0-only stores is compiled
@@ -767,167 +782,144 @@ __global__ __launch_bounds__(unit_threads(kTrav), kTrav == kUnitPerRay ? 4 : 6) 
 // disabled lane) and, for C = 1, never leave.  Every wave here runs
 // straight through, and its lane-dependent branches rejoin before the next
 // cross-lane operation.
-template <bool kStats, bool kSamples>
-__global__ __launch_bounds__(kTraceThreads, 5) void k_render_chunks(SceneView S, UnitLaunch U, int chunks) {
-  extern __shared__ uint32_t lane_stacks[];
-  const int lane = threadIdx.x & 63;
-  uint32_t* lane_stack = lane_stacks + threadIdx.x;
-  constexpr int kPer = kStats ? 3 : 1;
-  const uint64_t units = (uint64_t)U.pose_count * (uint64_t)U.omm_count;
-  const uint64_t tasks = units * (uint64_t)chunks;
-  const uint64_t t = (uint64_t)xcd_logical_block(blockIdx.x, gridDim.x) * (kTraceThreads / 64) +
-                     (uint64_t)(threadIdx.x >> 6);
-  if (t >= tasks) return;  // whole wave
-  const uint32_t n = (uint32_t)U.spp;
-  const float inv = 1.0f / (float)n;
-  const uint64_t uq = t / (uint64_t)chunks;
-  const uint32_t j = (uint32_t)(t - uq * (uint64_t)chunks);
-  int p, i;
-  uint64_t out;
-  locate_unit(U, uq, &p, &i, &out);
-  const uint32_t s = j * 64u + (uint32_t)lane;
-  const bool active = s < n;
-  float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a, c2 = a;
-  if (active) {
-    const U4 rnd = sample_randoms(U.seed, U.eye, (uint32_t)i, U.sample_base + s, U.frame,
-                                  U.pose_base + (uint32_t)p);
-    const Ray ray = generate_ray(U.omms[i], U.poses[p], rnd);
-    const RayPre rp = precompute_ray(ray);
-    Hit h;
-    closest_hit(S, rp, lane_stack, (int)blockDim.x, h);
-    const V3 c = shade(S, h, ray.dx, ray.dy, ray.dz);
-    const bool hit = h.id != 0xffffffffu;
-    a = make_float4(c.x * inv, c.y * inv, c.z * inv, 0.0f);
-    if (kSamples) U.samples[U.sample_offsets[out] + s] = make_float4(c.x, c.y, c.z, hit ? h.t : -1.0f);
-    if (kStats) {
-      const float idp = hit ? 1.0f / (1.0f + h.t) : 0.0f;
-      b = make_float4(c.x * c.x, c.y * c.y, c.z * c.z, idp);
-      c2 = make_float4(idp * idp, hit ? 1.0f : 0.0f, 0.0f, 0.0f);
-    }
-  }
-  float4* slot = U.chunk_partial + ((uq * (uint64_t)chunks + j) * 64u + (uint64_t)lane) * kPer;
-  slot[0] = a;
-  if (kStats) {
-    slot[1] = b;
-    slot[2] = c2;
-  }
-  __threadfence();
-  uint32_t prev = 0;
-  if (lane == 0) prev = atomicAdd(U.chunk_done + uq, 1u);
-  prev = __builtin_amdgcn_readfirstlane(__shfl(prev, 0));
-  if (prev != (uint32_t)chunks - 1u) return;  // whole wave
-  __threadfence();
-  float r = 0.0f, gg = 0.0f, bb = 0.0f;
-  float sr = 0.0f, sg = 0.0f, sb = 0.0f, sd = 0.0f, sd2 = 0.0f, sh = 0.0f;
-  for (int q = 0; q < chunks; ++q) {
-    if (q * 64 + lane < (int)n) {
-      const float4* src = U.chunk_partial + ((uq * (uint64_t)chunks + (uint64_t)q) * 64u + (uint64_t)lane) * kPer;
-      const float4 v = src[0];
-      r = r + v.x;
-      gg = gg + v.y;
-      bb = bb + v.z;
-      if (kStats) {
-        const float4 w = src[1], x = src[2];
-        sr += w.x;
-        sg += w.y;
-        sb += w.z;
-        sd += w.w;
-        sd2 += x.x;
-        sh += x.y;
-      }
-    }
-  }
-  r = segment_sum(r, 64);
-  gg = segment_sum(gg, 64);
-  bb = segment_sum(bb, 64);
-  if (kStats) {
-    sr = segment_sum(sr, 64);
-    sg = segment_sum(sg, 64);
-    sb = segment_sum(sb, 64);
-    sd = segment_sum(sd, 64);
-    sd2 = segment_sum(sd2, 64);
-    sh = segment_sum(sh, 64);
-  }
-  if (lane == 0) {
-    U.colours[out] = make_float4(r, gg, bb, (float)n);
-    if (kStats) {
-      const float vr = fmaxf(sr * inv - r * r, 0.0f);
-      const float vg = fmaxf(sg * inv - gg * gg, 0.0f);
-      const float vb = fmaxf(sb * inv - bb * bb, 0.0f);
-      const float md = sd * inv;
-      U.stats[2 * out] = make_float4(vr, vg, vb, sh * inv);
-      U.stats[2 * out + 1] = make_float4(md, fmaxf(sd2 * inv - md * md, 0.0f), 0.0f, 0.0f);
-    }
-  }
+__device__ __forceinline__ uchar4 make_color(float4 c) {
+  return make_uchar4(encode_channel(c.x), encode_channel(c.y), encode_channel(c.z), 255);
 }
 
-// The same split launch for wave-packet traversal: the whole wave returns
-// together when past the last task, and nothing but the traversal sits
-// between the ray generation and the chunk store, which keeps register use
-// low (more resident waves).  Same per-lane chunk values, completion
-// counters and last-wave reduction as k_render_chunks (no statistics).
+// Lane 0: the unit's colour, and its pixel.
+__device__ __forceinline__ void put_unit(KernelArgs* K, uint32_t i, float r, float g, float b) {
+  const float4 c = make_float4(r, g, b, (float)(uint32_t)K->U.spp);
+  K->U.colours[i] = c;
+  if (K->U.frame_pixels && i < (uint32_t)K->U.frame_width) K->U.frame_pixels[i] = make_color(c);
+}
+
+constexpr uint32_t kTaskFloats = 3 * 64;   // of `partial`, per task
+
+__device__ __forceinline__ void put_partial(KernelArgs* K, uint32_t t, int lane, float r, float g, float b) {
+  float* slot = K->U.chunk_partial + (size_t)t * kTaskFloats + lane;
+  slot[0] = r;
+  slot[64] = g;
+  slot[128] = b;
+}
+
+// One wave per unit: bound by reading 12 bytes per sample.
+__global__ __launch_bounds__(kTraceThreads) void k_reduce_tasks(RenderArgs A) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t u = blockIdx.x * (kTraceThreads / 64) + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (u >= (uint32_t)A.U.omm_count) return;   // whole wave
+  const uint32_t n = (uint32_t)A.U.spp, chunks = A.chunks;
+  const float* src = A.U.chunk_partial + (size_t)u * chunks * kTaskFloats + lane;
+  float r = 0.0f, g = 0.0f, b = 0.0f;
+  const uint32_t whole = n / 64u;   // chunks in which this lane has a sample, the last one apart
+  uint32_t q = 0;
+  for (; q + 8u <= whole; q += 8u) {
+    float v[8][3];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) v[k][c] = src[(size_t)(q + k) * kTaskFloats + 64 * c];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      r = r + v[k][0];
+      g = g + v[k][1];
+      b = b + v[k][2];
+    }
+  }
+  for (; q < chunks; ++q)
+    if (q * 64u + (uint32_t)lane < n) {
+      r = r + src[(size_t)q * kTaskFloats];
+      g = g + src[(size_t)q * kTaskFloats + 64];
+      b = b + src[(size_t)q * kTaskFloats + 128];
+    }
+  r = segment_sum(r, 64);
+  g = segment_sum(g, 64);
+  b = segment_sum(b, 64);
+  if (lane == 0) put_unit(fresh_args(), A.U.order ? A.U.order[u] : u, r, g, b);
+}
+
+// The rays of a task one per lane (an LDS stack column per lane): lanes past n
+// skip the traversal.
+template <bool kSamples>
+__global__ __launch_bounds__(kTraceThreads, 5) void k_render_chunks(RenderArgs A) {
+  extern __shared__ uint32_t lane_stacks[];
+  const int lane = threadIdx.x & 63;
+  const uint32_t t = xcd_run_block(blockIdx.x, gridDim.x, 16u) * (kTraceThreads / 64) +
+                     (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (t >= A.tasks) return;  // whole wave
+  uint32_t u, j;
+  split_unit(t, A.chunks, A.chunk_magic, &u, &j);
+  const uint32_t i = A.U.order ? A.U.order[u] : u;
+  const uint32_t s = j * 64u + (uint32_t)lane;
+  float r = 0.0f, g = 0.0f, b = 0.0f;
+  if (s < (uint32_t)A.U.spp) {
+    const U4 rnd = sample_randoms(A.U.seed, A.U.eye, i, A.U.sample_base + s, A.U.frame, A.U.pose_base);
+    const Ray ray = generate_ray(A.U.omms[i], A.pose, rnd);
+    const RayPre rp = precompute_ray(ray);
+    Hit h;
+    closest_hit(A.S, rp, lane_stacks + threadIdx.x, (int)blockDim.x, h);
+    const V3 c = shade(A.S, h, ray.dx, ray.dy, ray.dz);
+    r = c.x * A.inv;
+    g = c.y * A.inv;
+    b = c.z * A.inv;
+    if (kSamples)
+      A.U.samples[A.U.sample_offsets[i] + s] = make_float4(c.x, c.y, c.z, h.id != 0xffffffffu ? h.t : -1.0f);
+  }
+  put_partial(fresh_args(), t, lane, r, g, b);
+}
+
+// The rays of a task as one packet, in workgroups of one wave.  kSplit: the
+// launch records its tasks' packet steps and, with a list from the last
+// launch's (split_flag), traces the listed tasks first, as several packets.
 template <bool kSamples, int kTrav, bool kSplit>
-__global__ __launch_bounds__(kTraceThreads, 6) void k_render_tasks(SceneView S, UnitLaunch U, int chunks) {
+__global__ __launch_bounds__(64, 6) void k_render_tasks(RenderArgs A) {
   extern __shared__ uint32_t task_lds[];
   const int lane = threadIdx.x & 63;
-  const uint64_t units = (uint64_t)U.pose_count * (uint64_t)U.omm_count;
-  const uint64_t tasks = units * (uint64_t)chunks;
-  // the wave index read once as uniform: task, unit and output indices go to scalar registers
-  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const uint64_t wv = (uint64_t)xcd_logical_block(blockIdx.x, gridDim.x) * (kTraceThreads / 64) + (uint64_t)wave;
+  const uint32_t wv = xcd_run_block(blockIdx.x, gridDim.x, 64u);
   // With a long-task split the first kSplitSubWaves waves trace the listed
   // tasks: 4 waves per tier-0 task (wave w: part w % 4 of tier-0 task w / 4),
   // then 2 per tier-1 task, then one per tier-2 task (whole); the rest every
   // other task in order.
-  const bool split = kSplit && U.split_flag != nullptr;
-  const uint64_t sub_waves = split ? (uint64_t)kSplitSubWaves : 0u;
-  uint64_t t;
+  const bool split = kSplit && A.U.split_flag != nullptr;
+  const uint32_t sub_waves = split ? (uint32_t)kSplitSubWaves : 0u;
+  uint32_t t;
   int part = -1, ways = 1;
-  uint32_t li = 0;   // completion counter of a split task
   if (wv < sub_waves) {
     constexpr uint32_t r0 = 4u * kSplit4Max, r1 = r0 + 2u * kSplit2Max;
-    const uint32_t w = (uint32_t)wv;
     uint32_t tier, k, first;
-    if (w < r0) {
+    if (wv < r0) {
       tier = 0u;
-      k = w >> 2;
-      part = (int)(w & 3u);
+      k = wv >> 2;
+      part = (int)(wv & 3u);
       ways = 4;
       first = 0u;
-    } else if (w < r1) {
+    } else if (wv < r1) {
       tier = 1u;
-      k = (w - r0) >> 1;
-      part = (int)((w - r0) & 1u);
+      k = (wv - r0) >> 1;
+      part = (int)((wv - r0) & 1u);
       ways = 2;
       first = kSplit4Max;
     } else {
       tier = 2u;
-      k = w - r1;
+      k = wv - r1;
       first = kSplit4Max + kSplit2Max;
     }
-    const uint32_t listed = (uint32_t)__builtin_amdgcn_readfirstlane((int)U.split_count[tier]);
+    const uint32_t listed = (uint32_t)__builtin_amdgcn_readfirstlane((int)A.U.split_count[tier]);
     if (k >= listed) return;  // whole wave
-    t = (uint32_t)__builtin_amdgcn_readfirstlane((int)U.split_list[first + k]);
-    li = first + k;
+    t = (uint32_t)__builtin_amdgcn_readfirstlane((int)A.U.split_list[first + k]);
   } else {
     t = wv - sub_waves;
-    if (t >= tasks) return;  // whole wave
-    if (split && __builtin_amdgcn_readfirstlane((int)U.split_flag[t]) != 0) return;  // traced listed
+    if (t >= A.tasks) return;  // whole wave
+    if (split && __builtin_amdgcn_readfirstlane((int)A.U.split_flag[t]) != 0) return;  // traced listed
   }
-  const uint32_t n = (uint32_t)U.spp;
-  const float inv = 1.0f / (float)n;
-  const uint64_t uq = t / (uint64_t)chunks;
-  const uint32_t j = (uint32_t)(t - uq * (uint64_t)chunks);
-  int p, i;
-  uint64_t out;
-  locate_unit(U, uq, &p, &i, &out);
+  uint32_t u, j;
+  split_unit(t, A.chunks, A.chunk_magic, &u, &j);
+  const uint32_t i = (uint32_t)__builtin_amdgcn_readfirstlane((int)(A.U.order ? A.U.order[u] : u));
   const uint32_t s = j * 64u + (uint32_t)lane;
-  const bool active = s < n;
+  const bool active = s < (uint32_t)A.U.spp;
   Ray ray;
   if (active) {
-    const U4 rnd = sample_randoms(U.seed, U.eye, (uint32_t)i, U.sample_base + s, U.frame,
-                                  U.pose_base + (uint32_t)p);
-    ray = generate_ray(U.omms[i], U.poses[p], rnd);
+    const U4 rnd = sample_randoms(A.U.seed, A.U.eye, i, A.U.sample_base + s, A.U.frame, A.U.pose_base);
+    ray = generate_ray(A.U.omms[i], A.pose, rnd);
   } else {
     ray.ox = ray.oy = ray.oz = 0.0f;
     ray.dx = ray.dy = 0.0f;
@@ -935,7 +927,6 @@ __global__ __launch_bounds__(kTraceThreads, 6) void k_render_tasks(SceneView S, 
     ray.tmin = 0.0f;
     ray.tmax = 1.0f;
   }
-  const RayPre rp = precompute_ray(ray);
   // A split packet traces the lanes whose rays rank part * 64 / ways ..
   // (part + 1) * 64 / ways - 1 by elevation (the direction's y, ties by
   // lane): rays of neighbouring elevation fan out less than the whole chunk.
@@ -950,49 +941,36 @@ __global__ __launch_bounds__(kTraceThreads, 6) void k_render_tasks(SceneView S, 
   }
   Hit h;
   uint32_t w_steps = 0, w_tris = 0;
-  packet_hits<kTrav>(S, ray, rp, mine, task_lds, h, w_steps, w_tris);
-  if (U.packet_counts && lane == 0) {
-    atomicAdd(U.packet_counts, (unsigned long long)w_steps);
-    atomicAdd(U.packet_counts + 1, (unsigned long long)w_tris);
+  {
+    const SceneView S = walk_view(fresh_args());
+    packet_hits<kTrav>(S, ray, precompute_ray(ray), mine, task_lds, h, w_steps, w_tris);
   }
-  if (kSplit && U.split_cost && lane == 0) atomicAdd(U.split_cost + t, w_steps);
-  float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  KernelArgs* K = fresh_args();
+  if (K->U.packet_counts && lane == 0) {
+    atomicAdd(K->U.packet_counts, (unsigned long long)w_steps);
+    atomicAdd(K->U.packet_counts + 1, (unsigned long long)w_tris);
+  }
+  if (kSplit && K->U.split_cost && lane == 0) atomicAdd(K->U.split_cost + t, w_steps);
+  float r = 0.0f, g = 0.0f, b = 0.0f;
   if (mine) {
-    const V3 c = shade(S, h, ray.dx, ray.dy, ray.dz);
-    a = make_float4(c.x * inv, c.y * inv, c.z * inv, 0.0f);
+    const V3 c = shade(K->S.cols, K->S.texels, K->S.textures, K->S.sky_mode, h, ray.dx, ray.dy, ray.dz);
+    r = c.x * K->inv;
+    g = c.y * K->inv;
+    b = c.z * K->inv;
     if (kSamples)
-      U.samples[U.sample_offsets[out] + s] = make_float4(c.x, c.y, c.z, h.id != 0xffffffffu ? h.t : -1.0f);
+      K->U.samples[K->U.sample_offsets[i] + s] = make_float4(c.x, c.y, c.z, h.id != 0xffffffffu ? h.t : -1.0f);
+  }
+  if (!kSplit && K->chunks == 1u) {
+    // the unit's only chunk
+    r = segment_sum(0.0f + r, 64);
+    g = segment_sum(0.0f + g, 64);
+    b = segment_sum(0.0f + b, 64);
+    if (lane == 0) put_unit(K, i, r, g, b);
+    return;
   }
   // a split packet writes its own lanes' terms; the other packets of its
   // task write the rest
-  if (part < 0 || mine) U.chunk_partial[(uq * (uint64_t)chunks + j) * 64u + (uint64_t)lane] = a;
-  __threadfence();
-  if (part >= 0) {
-    // the last of the task's split packets to finish completes the task
-    uint32_t done = 0;
-    if (lane == 0) done = atomicAdd(U.split_sub_done + li, 1u);
-    done = __builtin_amdgcn_readfirstlane(__shfl(done, 0));
-    if (done != (uint32_t)ways - 1u) return;  // whole wave
-    __threadfence();
-  }
-  uint32_t prev = 0;
-  if (lane == 0) prev = atomicAdd(U.chunk_done + uq, 1u);
-  prev = __builtin_amdgcn_readfirstlane(__shfl(prev, 0));
-  if (prev != (uint32_t)chunks - 1u) return;  // whole wave
-  __threadfence();
-  float r = 0.0f, gg = 0.0f, bb = 0.0f;
-  for (int q = 0; q < chunks; ++q) {
-    if (q * 64 + lane < (int)n) {
-      const float4 v = U.chunk_partial[(uq * (uint64_t)chunks + (uint64_t)q) * 64u + (uint64_t)lane];
-      r = r + v.x;
-      gg = gg + v.y;
-      bb = bb + v.z;
-    }
-  }
-  r = segment_sum(r, 64);
-  gg = segment_sum(gg, 64);
-  bb = segment_sum(bb, 64);
-  if (lane == 0) U.colours[out] = make_float4(r, gg, bb, (float)n);
+  if (part < 0 || mine) put_partial(K, t, lane, r, g, b);
 }
 
 // Failure-handling probe of the packet traversal's partial-wave guard: one
@@ -1014,14 +992,13 @@ __global__ __launch_bounds__(64) void k_packet_guard_probe(SceneView S, const Ra
 }
 
 // Long-task split plan, one workgroup launched before the task kernel: it
-// clears the units' completion counters, takes a histogram of the last
+// takes a histogram of the last
 // launch's per-task packet steps (bins of 8 steps, the last one open), and
 // picks each tier's threshold: the smallest multiple of 8 steps at or above
 // the tier's minimum with at most the tiers' combined room (tier 0: 128
 // tasks, tiers 0-1: 1,024, tiers 0-2: 3,072) at or above it (none when even
 // the open top bin holds more).  It lists the tasks by tier and flags them,
-// and clears the split packets' completion counters and every task's step
-// count for this launch to fill in.
+// and clears every task's step count for this launch to fill in.
 constexpr int kSplitPlanThreads = 1024;
 constexpr int kSplitPlanPer = 16;   // step counts a thread holds at once
 static_assert(kSplitBins <= kSplitPlanThreads, "one thread per histogram bin");
@@ -1034,16 +1011,12 @@ __device__ __forceinline__ uint32_t split_threshold(uint32_t over, uint32_t min_
 __global__ __launch_bounds__(kSplitPlanThreads) void k_split_plan(uint32_t* __restrict__ cost, uint64_t tasks,
                                                                    uint32_t* __restrict__ flag,
                                                                    uint32_t* __restrict__ list,
-                                                                   uint32_t* __restrict__ count,
-                                                                   uint32_t* __restrict__ sub_done,
-                                                                   uint32_t* __restrict__ unit_done, uint64_t units) {
+                                                                   uint32_t* __restrict__ count) {
   __shared__ uint32_t hist[kSplitBins];
   __shared__ uint32_t listed[3];
   const uint32_t tid = threadIdx.x;
   for (uint32_t b = tid; b < (uint32_t)kSplitBins; b += kSplitPlanThreads) hist[b] = 0u;
   if (tid < 3u) listed[tid] = 0u;
-  for (uint32_t i = tid; i < (uint32_t)kSplitSubMax; i += kSplitPlanThreads) sub_done[i] = 0u;
-  for (uint64_t u = tid; u < units; u += kSplitPlanThreads) unit_done[u] = 0u;
   __syncthreads();
   // a round's loads are all issued before its histogram updates; only tasks
   // of at least kSplitEarlyMinSteps enter the histogram (shorter ones are
@@ -1171,10 +1144,6 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_rays(SceneView S, const
   tbb[r] = make_float4(h.t, h.b1, h.b2, 0.0f);
 }
 
-__device__ __forceinline__ uchar4 make_color(float4 c) {
-  return make_uchar4(encode_channel(c.x), encode_channel(c.y), encode_channel(c.z), 255);
-}
-
 // One pixel of a regular camera per thread: primary ray, closest hit
 // (per-ray LDS stack), shading or sky, make_color.  rays (nullable) receives
 // the generated rays.
@@ -1272,19 +1241,6 @@ static UnitsKernel units_kernel_of(const UnitLaunch& U) {
   return units_kernel_variant<kUnitPacket>(U);
 }
 
-static void launch_chunks(const UnitLaunch& U, const SceneView& v, int blocks, size_t lds, int chunks,
-                          hipStream_t stream) {
-  const dim3 grid(blocks), block(kTraceThreads);
-  if (U.stats && U.samples)
-    hipLaunchKernelGGL((k_render_chunks<true, true>), grid, block, lds, stream, v, U, chunks);
-  else if (U.stats)
-    hipLaunchKernelGGL((k_render_chunks<true, false>), grid, block, lds, stream, v, U, chunks);
-  else if (U.samples)
-    hipLaunchKernelGGL((k_render_chunks<false, true>), grid, block, lds, stream, v, U, chunks);
-  else
-    hipLaunchKernelGGL((k_render_chunks<false, false>), grid, block, lds, stream, v, U, chunks);
-}
-
 static int device_cus() {
   static int cus = 0;
   if (cus == 0) {
@@ -1325,10 +1281,15 @@ int render_units_capacity(const DeviceScene& scene, const UnitLaunch& U_in) {
   return std::max(1, device_cus() * per_cu * threads / kTraceThreads);
 }
 
+static uint32_t magic_of(int n) { return (uint32_t)std::min<uint64_t>(0xffffffffull, (1ull << 32) / (uint64_t)n); }
+
 bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipStream_t stream, std::string* err) {
   UnitLaunch U = U_in;
   const uint64_t units = (uint64_t)U.pose_count * (uint64_t)U.omm_count;
-  if (units == 0) return true;
+  if (units == 0) {
+    if (U.traced) (void)hipEventRecord(U.traced, stream);
+    return true;
+  }
   if (units > kMaxLaunchUnits) {
     if (err) *err = "render_units: too many units for one launch";
     return false;
@@ -1349,79 +1310,81 @@ bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipSt
   }
   const int capacity = render_units_capacity(scene, U);
   const SceneView v = view_of(scene);
-  // Split launch: uniform counts and fewer units than two per wave slot of
-  // the device (a single pose, typically), when the caller gave scratch: each
-  // unit's 64-sample chunks are tasks of their own, one wave each.  With
-  // per-ray traversal or statistics, units of 32 samples or fewer stay in the
-  // unit kernel, which packs two or more of them into a wave's lanes (a
-  // per-ray task would leave the other lanes idle); the packet task kernel
-  // takes any count (a single pose still renders sooner that way).  The slots
-  // are counted at the kernels' launch bound (5 blocks of 4 waves per CU) or
-  // the unit kernel's occupancy if higher, not lowered by the LDS the per-ray
-  // stack takes: a deep tree's per-ray stack cuts the persistent unit kernel
-  // to two blocks per CU, which leaves a single pose badly balanced.
+  RenderArgs A{};
+  A.S = v;
+  A.U = U;
+  if (U.host_pose) A.pose = *U.host_pose;
+  A.omm_magic = magic_of(U.omm_count);
+  // Split launch: one pose, a uniform count and fewer units than two per wave
+  // slot of the device, when the caller gave scratch: each unit's 64-sample
+  // chunks are tasks of their own, one wave each.  With per-ray traversal
+  // units of 32 samples or fewer stay in the unit kernel, which packs two or
+  // more of them into a wave's lanes (a per-ray task would leave the other
+  // lanes idle); the packet task kernel takes any count (a single pose still
+  // renders sooner that way).  The slots are counted at the kernels' launch
+  // bound (5 blocks of 4 waves per CU) or the unit kernel's occupancy if
+  // higher, not lowered by the LDS the per-ray stack takes: a deep tree's
+  // per-ray stack cuts the unit kernel to two blocks per CU, which leaves a
+  // single pose badly balanced.
   const uint64_t chunks = U.spp > 64 ? ((uint64_t)U.spp + 63u) / 64u : 1u;
   const uint64_t resident_waves = (uint64_t)std::max(capacity, device_cus() * 5) * (kTraceThreads / 64);
-  const uint64_t per_chunk = U.stats ? 3u : 1u;
-  const bool packet_tasks = U.traversal != kUnitPerRay && !U.stats;
-  if (g_split && !U.omm_counts && !U.unit_counts && (U.spp > 32 || packet_tasks) && units < 2 * resident_waves &&
-      U.chunk_partial && U.chunk_done && units * chunks <= 0xffffffffull - 65536ull &&
-      units * chunks * 64u * per_chunk <= U.chunk_partial_cap && units <= U.chunk_done_cap) {
-    const uint64_t tasks = units * chunks;
-    if (packet_tasks && tasks / (kTraceThreads / 64) < 0x7fffffffull - (uint64_t)kSplitSubWaves) {
-      // wave packets: the non-persistent task kernel, one wave per chunk
-      UnitLaunch T = U;
-      const bool have_split = U.split_cost && U.split_flag && U.split_list && U.split_count && U.split_sub_done &&
-                              U.split_tasks == tasks;
+  const bool packet_tasks = U.traversal != kUnitPerRay;
+  const uint64_t tasks = units * chunks;
+  if (g_split && U.host_pose && !U.omm_counts && !U.unit_counts && !U.stats && (U.spp > 32 || packet_tasks) &&
+      units < 2 * resident_waves && U.chunk_partial && tasks <= 0x7fffffffull - (uint64_t)kSplitSubWaves &&
+      tasks * kTaskFloats <= U.chunk_partial_cap) {
+    A.chunks = (uint32_t)chunks;
+    A.chunk_magic = magic_of((int)chunks);
+    A.tasks = (uint32_t)tasks;
+    A.inv = 1.0f / (float)(uint32_t)U.spp;
+    bool reduce = chunks > 1;
+    if (packet_tasks) {
+      const bool have_split = U.split_cost && U.split_flag && U.split_list && U.split_count && U.split_tasks == tasks;
       if (have_split && U.split_plan) {
-        // the plan kernel also clears the units' completion counters
         hipLaunchKernelGGL(k_split_plan, dim3(1), dim3(kSplitPlanThreads), 0, stream, U.split_cost, tasks,
-                           U.split_flag, U.split_list, U.split_count, U.split_sub_done, U.chunk_done, units);
+                           U.split_flag, U.split_list, U.split_count);
       } else {
-        hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, U.chunk_done,
-                           (uint32_t)units, 0u);
-        T.split_flag = nullptr;
+        A.U.split_flag = nullptr;
         if (have_split)  // no steps of these tasks yet: record them, split nothing
           hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((tasks + 255) / 256)), dim3(256), 0, stream, U.split_cost,
                              (uint32_t)tasks, 0u);
         else
-          T.split_cost = nullptr;
+          A.U.split_cost = nullptr;
       }
-      const uint64_t waves = tasks + (T.split_flag ? (uint64_t)kSplitSubWaves : 0u);
-      const dim3 grid((unsigned)((waves + (kTraceThreads / 64) - 1) / (kTraceThreads / 64))), block(kTraceThreads);
       const bool wide = U.traversal == kUnitPacketWide;
       constexpr int kW = kUnitPacketWide, kP = kUnitPacket;
       // the variant without the split's code keeps the registers of the plain task kernel
       auto kernel = U.samples ? (wide ? k_render_tasks<true, kW, false> : k_render_tasks<true, kP, false>)
                               : (wide ? k_render_tasks<false, kW, false> : k_render_tasks<false, kP, false>);
-      if (T.split_cost)
+      if (A.U.split_cost) {
         kernel = U.samples ? (wide ? k_render_tasks<true, kW, true> : k_render_tasks<true, kP, true>)
                            : (wide ? k_render_tasks<false, kW, true> : k_render_tasks<false, kP, true>);
-      hipLaunchKernelGGL(kernel, grid, block, lds, stream, v, T, (int)chunks);
+        reduce = true;
+      }
+      const uint64_t waves = tasks + (A.U.split_flag ? (uint64_t)kSplitSubWaves : 0u);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)waves), dim3(64), units_lds_bytes(scene, U.traversal, 1), stream, A);
       g_last_kernel = "k_render_tasks";
-      return check_launch("render_tasks", err);
+    } else {
+      // per-ray traversal: an LDS stack column per lane
+      const unsigned grid = (unsigned)((tasks + (kTraceThreads / 64) - 1) / (kTraceThreads / 64));
+      if (U.samples)
+        hipLaunchKernelGGL(k_render_chunks<true>, dim3(grid), dim3(kTraceThreads), lds, stream, A);
+      else
+        hipLaunchKernelGGL(k_render_chunks<false>, dim3(grid), dim3(kTraceThreads), lds, stream, A);
+      reduce = true;
+      g_last_kernel = "k_render_chunks";
     }
-    // per-ray traversal: the chunk kernel, one wave per chunk, an LDS stack
-    // column per lane
-    const size_t chunk_lds = stack_bytes(scene);
-    if (chunk_lds > 160 * 1024) {
-      if (err) *err = "render_chunks: BVH too deep for the LDS traversal stack";
+    if (U.traced && hipEventRecord(U.traced, stream) != hipSuccess) {
+      if (err) *err = "render_tasks: event";
       return false;
     }
-    if (tasks / (kTraceThreads / 64) >= 0x7fffffffull) {
-      if (err) *err = "render_chunks: too many chunks for one launch";
-      return false;
-    }
-    const int chunk_blocks = (int)((tasks + (kTraceThreads / 64) - 1) / (kTraceThreads / 64));
-    hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, stream, U.chunk_done,
-                       (uint32_t)units, 0u);
-    launch_chunks(U, v, chunk_blocks, chunk_lds, (int)chunks, stream);
-    g_last_kernel = "k_render_chunks";
-    return check_launch("render_chunks", err);
+    if (reduce)
+      hipLaunchKernelGGL(k_reduce_tasks, dim3((unsigned)((units + 3) / 4)), dim3(kTraceThreads), 0, stream, A);
+    if (U.frame_done) *U.frame_done = U.frame_pixels != nullptr;
+    return check_launch("render_tasks", err);
   }
   // Units per wave: as given, or (0) as many as leave four waves for every
   // resident slot, at most auto_grab_max, but enough to fill a wave's lanes.
-  RenderArgs A{v, U, 0, 0, 1};
   if (A.U.units_per_grab <= 0) {
     uint64_t fill = 1;
     if (one_pass(U))
@@ -1430,7 +1393,6 @@ bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipSt
         fill, std::min<uint64_t>((uint64_t)std::max(U.auto_grab_max, 1), units / (4 * resident_waves)));
   }
   A.U.units_per_grab = std::min(A.U.units_per_grab, kMaxUnitsPerGrab);
-  A.omm_magic = (uint32_t)std::min<uint64_t>(0xffffffffull, (1ull << 32) / (uint64_t)U.omm_count);
   const int threads = unit_threads(U.traversal);
   const uint64_t per_block = (uint64_t)A.U.units_per_grab * (uint64_t)(threads / 64);
   A.blocks = (uint32_t)((units + per_block - 1) / per_block);
@@ -1443,6 +1405,7 @@ bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipSt
                    : A.blocks;
   hipLaunchKernelGGL(units_kernel_of(U), dim3(grid), dim3(threads), units_lds_bytes(scene, U.traversal, threads / 64),
                      stream, A);
+  if (U.traced) (void)hipEventRecord(U.traced, stream);
   g_last_kernel = "k_render_units";
   return check_launch("render_units", err);
 }

@@ -189,3 +189,37 @@ def test_unit_grid_shapes(lib, tmp_path, grab, blocks, counts):
     finally:
         lib.setRenderTuning(0, 0)
         er.set_sample_counts(lib, None)
+
+
+@pytest.mark.parametrize("spp", [1, 64, 65, 512, 513, 575, 577, 1100])
+@pytest.mark.parametrize("width", [40, 71, 90])
+@pytest.mark.parametrize("split", [0, 1])
+def test_frame_chunks(lib, tmp_path, spp, width, split):
+    """renderFrame's 64-sample chunks on different waves, around the reduction's
+    runs of eight chunks: colours, and the frame row of single_dimension_fast
+    narrower and wider than the eye (pixels beyond it stay as they were)."""
+    pos, col = soup(300, 16)
+    omm = eye_of(random_axes(71, 10), -2.0 * random_axes(71, 10), 0.2)
+    sc = scenes.Scene([scenes.Mesh("m", pos, np.arange(len(pos), dtype=np.uint32).reshape(-1, 3), col)],
+                      eyes=[scenes.Eye("eye", omm)])
+    lib.loadGlTFscene(str(scenes.write_gltf(tmp_path, "s", sc)).encode())
+    er.gotoFirstCompoundEye(lib)
+    er.set_ommatidia_np(lib, omm)
+    lib.setCurrentEyeSamplesPerOmmatidium(spp)
+    lib.setCameraPose(0, 0, 0, 0, 0, 0)
+    er.setRenderSize(lib, width, 2)
+    lib.setTaskSplit(split)
+    try:
+        want = oracle.OracleScene.from_scene(sc)
+        for frame in range(3):
+            assert lib.renderFrame() >= 0, er.last_error(lib)
+            ref = want.render(omm, er.pose_np(lib), spp=spp, frame=frame)["colour_gpu_order"][0]
+            assert lib.getLastRenderKernel() == b"k_render_tasks"
+            assert np.array_equal(er.colours_np(lib), ref)
+            pixels = np.array(lib.getFramePointer(), copy=True).reshape(2, width, 4)
+            n = min(width, 71)
+            assert np.array_equal(pixels[0, :n], oracle.make_color(ref)[:n])
+            assert not pixels[0, n:].any() and not pixels[1].any()
+    finally:
+        lib.setTaskSplit(2)
+        er.setRenderSize(lib, 400, 400)
