@@ -42,6 +42,8 @@ struct EyeState {
   std::string shader = "single_dimension_fast";
   Ommatidium* d_omms = nullptr;
   size_t d_omms_cap = 0;
+  Cone* d_cones = nullptr;               // of d_omms
+  size_t d_cones_cap = 0;
   uint32_t* d_offsets = nullptr;
   size_t d_offsets_cap = 0;
   uint32_t* d_counts = nullptr;          // per-ommatidium sample counts (when counts are set)
@@ -241,6 +243,7 @@ void free_scene() {
   s.d_textures = nullptr;
   for (EyeState& e : s.eyes) {
     if (e.d_omms) (void)hipFree(e.d_omms);
+    if (e.d_cones) (void)hipFree(e.d_cones);
     if (e.d_offsets) (void)hipFree(e.d_offsets);
     if (e.d_samples) (void)hipFree(e.d_samples);
     if (e.d_colours) (void)hipFree(e.d_colours);
@@ -315,9 +318,12 @@ void upload_eye(EyeState& e) {
   std::vector<uint32_t> order;
   if (e.omm_dirty) {
     ensure_device(&e.d_omms, &e.d_omms_cap, n);
+    ensure_device(&e.d_cones, &e.d_cones_cap, n);
     if (n)
       hip_check(hipMemcpyAsync(e.d_omms, e.omms.data(), sizeof(Ommatidium) * n, hipMemcpyHostToDevice, s.stream),
                 "upload ommatidia");
+    std::string err;
+    if (!launch_cones(e.d_omms, (int)n, e.d_cones, s.stream, &err)) throw std::runtime_error(err);
     // Units are processed in the order of (position cell, axis Morton code):
     // waves running at the same time trace neighbouring view directions from
     // the same place and share BVH nodes in cache.  Cells are 1 scene unit (or
@@ -407,6 +413,7 @@ UnitLaunch unit_launch_of(EyeState& e, const Pose* d_poses, int pose_count) {
   State& s = st();
   UnitLaunch U;
   U.omms = e.d_omms;
+  U.cones = e.d_cones;
   U.omm_count = (int)e.omms.size();
   U.poses = d_poses;
   U.pose_count = pose_count;

@@ -61,14 +61,6 @@ struct U4 {
   uint32_t a, b, c, d;
 };
 
-EYE_HD uint32_t mulhi32(uint32_t a, uint32_t b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __umulhi(a, b);
-#else
-  return (uint32_t)(((uint64_t)a * (uint64_t)b) >> 32);
-#endif
-}
-
 EYE_HD U4 philox4x32_10(U4 ctr, uint32_t k0, uint32_t k1) {
   const uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u;
   const uint32_t W0 = 0x9E3779B9u, W1 = 0xBB67AE85u;
@@ -76,13 +68,13 @@ EYE_HD U4 philox4x32_10(U4 ctr, uint32_t k0, uint32_t k1) {
 #pragma unroll
 #endif
   for (int r = 0; r < 10; ++r) {
-    const uint32_t hi0 = mulhi32(M0, ctr.a), lo0 = M0 * ctr.a;
-    const uint32_t hi1 = mulhi32(M1, ctr.c), lo1 = M1 * ctr.c;
+    // whole products: one 64-bit multiply each
+    const uint64_t p0 = (uint64_t)M0 * ctr.a, p1 = (uint64_t)M1 * ctr.c;
     U4 n;
-    n.a = hi1 ^ ctr.b ^ k0;
-    n.b = lo1;
-    n.c = hi0 ^ ctr.d ^ k1;
-    n.d = lo0;
+    n.a = (uint32_t)(p1 >> 32) ^ ctr.b ^ k0;
+    n.b = (uint32_t)p1;
+    n.c = (uint32_t)(p0 >> 32) ^ ctr.d ^ k1;
+    n.d = (uint32_t)p0;
     ctr = n;
     k0 += W0;
     k1 += W1;
@@ -108,20 +100,43 @@ EYE_HD float box_muller(uint32_t r0, uint32_t r1) {
 constexpr float kFwhmSdRatio = 2.35482004503094938f;
 
 // Rodrigues rotation of `p` by `angle` about `k` (k not normalised here, as in
-// libEyeRenderer3/shaders.cu:648-651).
-EYE_HD V3 rotate_point(V3 p, float angle, V3 k) {
+// libEyeRenderer3/shaders.cu:648-651), given cross(k, p) and dot(k, p).
+EYE_HD V3 rotate_point(V3 p, float angle, V3 k, V3 k_cross_p, float k_dot_p) {
   float s, c;
   det_sincos(angle, &s, &c);
-  return (c * p + s * cross(k, p)) + ((1.0f - c) * dot(k, p)) * k;
+  return (c * p + s * k_cross_p) + ((1.0f - c) * k_dot_p) * k;
+}
+
+// What the rays of one ommatidium share, 64 bytes: its axis, the perpendicular
+// about which rays are splayed and its products with the axis, the cone's
+// standard deviation and the rays' start in the eye's frame.
+struct Cone {
+  float dx, dy, dz, focal_offset;
+  float kx, ky, kz, sd;        // perpendicular
+  float cx, cy, cz, along;     // perpendicular x axis, perpendicular . axis
+  float ox, oy, oz, unused;
+};
+
+EYE_HD Cone cone_of(const Ommatidium& o) {
+  const V3 axis = v3(o.dx, o.dy, o.dz);
+  V3 perp = cross(v3(0.0f, 1.0f, 0.0f), axis);
+  perp = (perp.x + perp.y + perp.z == 0.0f) ? v3(0.0f, 0.0f, 1.0f) : normalize(perp);
+  const V3 side = cross(perp, axis);
+  const V3 start = v3(o.px, o.py, o.pz) - normalize(axis) * o.focal_offset;
+  Cone c;
+  c.dx = o.dx; c.dy = o.dy; c.dz = o.dz; c.focal_offset = o.focal_offset;
+  c.kx = perp.x; c.ky = perp.y; c.kz = perp.z; c.sd = o.acceptance / kFwhmSdRatio;
+  c.cx = side.x; c.cy = side.y; c.cz = side.z; c.along = dot(perp, axis);
+  c.ox = start.x; c.oy = start.y; c.oz = start.z; c.unused = 0.0f;
+  return c;
 }
 
 // libEyeRenderer3/shaders.cu:652-662: splay the axis away from itself by
-// `splay` about a perpendicular, then spin it by `spin` about the axis.
-EYE_HD V3 offset_ray(float spin, float splay, V3 axis) {
-  V3 perp = cross(v3(0.0f, 1.0f, 0.0f), axis);
-  perp = (perp.x + perp.y + perp.z == 0.0f) ? v3(0.0f, 0.0f, 1.0f) : normalize(perp);
-  const V3 splayed = rotate_point(axis, splay, perp);
-  return rotate_point(splayed, spin, axis);
+// `splay` about the perpendicular, then spin it by `spin` about the axis.
+EYE_HD V3 offset_ray(float spin, float splay, const Cone& c) {
+  const V3 axis = v3(c.dx, c.dy, c.dz), perp = v3(c.kx, c.ky, c.kz), side = v3(c.cx, c.cy, c.cz);
+  const V3 splayed = rotate_point(axis, splay, perp, side, c.along);
+  return rotate_point(splayed, spin, axis, cross(axis, splayed), dot(axis, splayed));
 }
 
 // Random stream of one sample: key (seed, eye), counter (ommatidium, sample,
@@ -137,13 +152,11 @@ EYE_HD U4 sample_randoms(uint32_t seed, uint32_t eye, uint32_t omm, uint32_t sam
 
 // Ray of one sample of one ommatidium in world space
 // (libEyeRenderer3/shaders.cu:664-723).
-EYE_HD Ray generate_ray(const Ommatidium& o, const Pose& p, U4 rnd) {
-  const float sd = o.acceptance / kFwhmSdRatio;
-  const float splay = box_muller(rnd.a, rnd.b) * sd;
+EYE_HD Ray generate_ray(const Cone& o, const Pose& p, U4 rnd) {
+  const float splay = box_muller(rnd.a, rnd.b) * o.sd;
   const float spin = u01_open0(rnd.c) * kPiF;
-  const V3 axis = v3(o.dx, o.dy, o.dz);
-  const V3 rdir = offset_ray(spin, splay, axis);
-  const V3 rpos = v3(o.px, o.py, o.pz) - normalize(axis) * o.focal_offset;
+  const V3 rdir = offset_ray(spin, splay, o);
+  const V3 rpos = v3(o.ox, o.oy, o.oz);
   const V3 X = v3(p.x[0], p.x[1], p.x[2]);
   const V3 Y = v3(p.y[0], p.y[1], p.y[2]);
   const V3 Z = v3(p.z[0], p.z[1], p.z[2]);
@@ -338,9 +351,18 @@ EYE_HD float fold_coord(float u, int mode) {
   return u - floorf(u);
 }
 
+// b / 255, the rounded quotient of every byte, as a product with 1 / 255 in two
+// floats (a division is 12 instructions, and a filtered texel takes 12).
+constexpr float kInv255Hi = 3.9215688593685627e-3f;   // float(1 / 255)
+constexpr float kInv255Lo = -2.3191758236e-10f;       // float(1 / 255 - hi)
+EYE_HD float unit_byte(uint32_t b) {
+  const float f = (float)b;
+  return fmaf(f, kInv255Hi, f * kInv255Lo);
+}
+
 EYE_HD V3 texel_rgb(const uint32_t* texels, const TexView& t, int i, int j) {
   const uint32_t v = texels[t.first + (uint32_t)j * (uint32_t)t.width + (uint32_t)i];
-  return v3((float)(v & 0xffu) / 255.0f, (float)((v >> 8) & 0xffu) / 255.0f, (float)((v >> 16) & 0xffu) / 255.0f);
+  return v3(unit_byte(v & 0xffu), unit_byte((v >> 8) & 0xffu), unit_byte((v >> 16) & 0xffu));
 }
 
 // tex2D with normalised coordinates and normalised-float reads: point

@@ -52,24 +52,37 @@ __device__ __forceinline__ float first_f(float v) {
   return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
 
-// Wave-wide extremes on DPP moves (four within rows of 16 lanes, two across
-// rows): no LDS round trips and no address registers.
-template <int kCtrl, int kRows = 0xf>
-__device__ __forceinline__ float dpp_f(float v) {
-  const int i = __float_as_int(v);
-  return __int_as_float(__builtin_amdgcn_update_dpp(i, i, kCtrl, kRows, 0xf, false));
+// Wave-wide maxima of six values, each in its VGPR at once: six DPP maxima
+// per value (four within rows of 16 lanes, two across rows), the values taking
+// turns, which also keeps the two wait states between a write and its DPP read.
+// The compiler's form of one step is a copy, a wait, a DPP move, two
+// canonicalising maxima and the maximum: 435 VALU instructions for a packet's
+// bounds, 230 so.  Every lane of the wave takes part.
+__device__ __forceinline__ void wave_max6(float& a, float& b, float& c, float& d, float& e, float& f) {
+#define EYE_DPP_STEP(ctrl)                      \
+  "v_max_f32_dpp %0, %0, %0 " ctrl "\n\t"       \
+  "v_max_f32_dpp %1, %1, %1 " ctrl "\n\t"       \
+  "v_max_f32_dpp %2, %2, %2 " ctrl "\n\t"       \
+  "v_max_f32_dpp %3, %3, %3 " ctrl "\n\t"       \
+  "v_max_f32_dpp %4, %4, %4 " ctrl "\n\t"       \
+  "v_max_f32_dpp %5, %5, %5 " ctrl "\n\t"
+  asm volatile("s_nop 1\n\t"
+               EYE_DPP_STEP("quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf")
+               EYE_DPP_STEP("quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf")
+               EYE_DPP_STEP("row_half_mirror row_mask:0xf bank_mask:0xf")
+               EYE_DPP_STEP("row_mirror row_mask:0xf bank_mask:0xf")
+               EYE_DPP_STEP("row_bcast:15 row_mask:0xa bank_mask:0xf")
+               EYE_DPP_STEP("row_bcast:31 row_mask:0xc bank_mask:0xf")
+               "s_nop 1"
+               : "+v"(a), "+v"(b), "+v"(c), "+v"(d), "+v"(e), "+v"(f));
+#undef EYE_DPP_STEP
+  a = lane_f(a, 63);
+  b = lane_f(b, 63);
+  c = lane_f(c, 63);
+  d = lane_f(d, 63);
+  e = lane_f(e, 63);
+  f = lane_f(f, 63);
 }
-__device__ __forceinline__ float wave_max(float v) {
-  v = fmaxf(v, dpp_f<0xb1>(v));         // quad_perm 1 0 3 2
-  v = fmaxf(v, dpp_f<0x4e>(v));         // quad_perm 2 3 0 1
-  v = fmaxf(v, dpp_f<0x141>(v));        // row_half_mirror
-  v = fmaxf(v, dpp_f<0x140>(v));        // row_mirror
-  v = fmaxf(v, dpp_f<0x142, 0xa>(v));   // row_bcast15 into rows 1 and 3
-  v = fmaxf(v, dpp_f<0x143, 0xc>(v));   // row_bcast31 into rows 2 and 3
-  return lane_f(v, 63);
-}
-// The same for values of which only an order among the non-negative and -inf
-// is needed: as integers, which need no canonical form.
 template <int kCtrl, int kRows = 0xf>
 __device__ __forceinline__ int dpp_i(int i) {
   return __builtin_amdgcn_update_dpp(i, i, kCtrl, kRows, 0xf, false);
@@ -157,9 +170,9 @@ __device__ __forceinline__ void test_triangle(const PacketRay& r, const V3& a, c
   const float U = cx * by - cy * bx;
   const float V = ax * cy - ay * cx;
   const float W = bx * ay - by * ax;
-  if ((U < 0.0f || V < 0.0f || W < 0.0f) && (U > 0.0f || V > 0.0f || W > 0.0f)) return;
   const float det = U + V + W;
-  if (det == 0.0f) return;
+  // two signs among the edges, or none of any size
+  if ((fminf(fminf(U, V), W) < 0.0f) & (fmaxf(fmaxf(U, V), W) > 0.0f) | (det == 0.0f)) return;
   const float T = U * (r.sz * az) + V * (r.sz * bz) + W * (r.sz * cz);
   const float t = T / det;
   if (t >= r.tmin && (t < h.t || (t == h.t && id < h.id))) {
@@ -364,12 +377,13 @@ __device__ __forceinline__ void closest_hit_wide(const WideTree& T, const Ray& r
     a = in ? a : 0.0f;
     b = in ? b : 0.0f;
     const float margin = 8e-6f;   // slopes are below 1
-    B.a0 = first_f(-wave_max(-a) - margin);
-    B.a1 = first_f(wave_max(a) + margin);
-    B.b0 = first_f(-wave_max(-b) - margin);
-    B.b1 = first_f(wave_max(b) + margin);
-    B.reach = wave_max_depth(in ? k * size : 0.0f) * 1.0002f;
-    const float out = wave_max_depth(in ? far : 0.0f);
+    float a0 = -a, a1 = a, b0 = -b, b1 = b, reach = in ? k * size : 0.0f, out = in ? far : 0.0f;
+    wave_max6(a0, a1, b0, b1, reach, out);
+    B.a0 = first_f(-a0 - margin);
+    B.a1 = first_f(a1 + margin);
+    B.b0 = first_f(-b0 - margin);
+    B.b1 = first_f(b1 + margin);
+    B.reach = reach * 1.0002f;
     B.pad = 2.0f * kWidePad * out;
     // where the rays start: a negative tmin starts behind the origin
     const float back = fminf(rp.tmin, 0.0f);
@@ -379,12 +393,9 @@ __device__ __forceinline__ void closest_hit_wide(const WideTree& T, const Ray& r
     float oa1 = pu - B.a1 * pw, oa0 = B.a0 * pw - pu, ob1 = pv - B.b1 * pw, ob0 = B.b0 * pw - pv, nr = pw, fr = pw;
     // one start for all rays (samples of one ommatidium): no reductions
     if (__ballot(p.x != o0.x || p.y != o0.y || p.z != o0.z) != 0ull) {
-      oa0 = wave_max(oa0);
-      oa1 = wave_max(oa1);
-      ob0 = wave_max(ob0);
-      ob1 = wave_max(ob1);
-      nr = -wave_max(-nr);
-      fr = wave_max(fr);
+      nr = -nr;
+      wave_max6(oa0, oa1, ob0, ob1, nr, fr);
+      nr = -nr;
     }
     const float m = 8.0f * kWidePad * out;
     B.oa0 = first_f(oa0 + m);

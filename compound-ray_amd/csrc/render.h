@@ -50,6 +50,7 @@ constexpr uint64_t split_buffer_words(uint64_t tasks) { return 2 * tasks + (uint
 // per-sample buffer is needed.
 struct UnitLaunch {
   const Ommatidium* omms = nullptr;
+  const Cone* cones = nullptr;          // of the same ommatidia
   int omm_count = 0;
   const Pose* poses = nullptr;
   int pose_count = 1;
@@ -165,6 +166,8 @@ bool launch_camera_frame(const DeviceScene& scene, const CameraLaunch& C, uchar4
                          hipStream_t stream, std::string* err);
 
 // Rays of one eye at one pose, in (ommatidium, sample) order, 8 floats each.
+// cones[i] = cone_of(omms[i]).
+bool launch_cones(const Ommatidium* omms, int omm_count, Cone* cones, hipStream_t stream, std::string* err);
 bool launch_generate_rays(const EyeLaunch& L, Ray* rays, hipStream_t stream, std::string* err);
 
 // Closest hits of arbitrary rays: hit[i] = original triangle id or -1,
