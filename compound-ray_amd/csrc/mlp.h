@@ -46,10 +46,9 @@ class Mlp {
   // [0, n) of device arrays; *loss and grad are device outputs.
   bool loss_grad(const float* d_x, const float* d_t, int64_t n, float* d_loss, float* d_grad,
                  hipStream_t stream, std::string* err);
-  // One Adam step (beta1 0.9, beta2 0.999, eps 1e-8) with gradient d_grad.
-  bool adam_step(const float* d_grad, float lr, hipStream_t stream, std::string* err);
-  // Minibatch training over device arrays, rows shuffled per epoch with a
-  // seeded permutation; losses receives the mean loss of every epoch.
+  // Minibatch training over device arrays (Adam, beta1 0.9, beta2 0.999, eps
+  // 1e-8), rows shuffled per epoch with a seeded permutation; losses receives
+  // the mean loss of every epoch.
   bool train(const float* d_x, const float* d_t, int64_t n, int epochs, int batch, float lr, uint32_t seed,
              std::vector<float>* losses, hipStream_t stream, std::string* err);
   bool ready() const { return master_ != nullptr; }
@@ -57,17 +56,20 @@ class Mlp {
 
  private:
   bool pack(hipStream_t stream, std::string* err);
+  // Gradient partials of rows d_idx[0 .. n) (null: rows 0 .. n); returns the
+  // number of blocks.
+  int grad(const float* d_x, const float* d_t, const uint32_t* d_idx, int64_t n, hipStream_t stream);
+  // One Adam step on those rows; *d_loss receives their mean squared error.
+  bool train_step(const float* d_x, const float* d_t, const uint32_t* d_idx, int64_t n, float lr, float* d_loss,
+                  hipStream_t stream, std::string* err);
   float* master_ = nullptr;      // kMlpParams
   float* adam_m_ = nullptr;
   float* adam_v_ = nullptr;
   uint16_t* packed_ = nullptr;   // BF16 layouts for the kernels
   float* partial_ = nullptr;     // per-block gradient partials
   float* loss_partial_ = nullptr;
-  float* grad_ = nullptr;
-  float* loss_ = nullptr;
-  float* xb_ = nullptr;          // gathered minibatch
-  float* tb_ = nullptr;
-  int64_t batch_cap_ = 0;
+  static constexpr int kLossRing = 1024;
+  float* loss_ = nullptr;        // kLossRing, of the last batches
   uint32_t* perm_ = nullptr;
   int64_t perm_cap_ = 0;
   int64_t step_ = 0;
