@@ -499,6 +499,8 @@ double render_compound(EyeState& e, const Cam& c) {
     }
     bool rec = false, plan = false;
     split_choice(e, &rec, &plan);
+    // tasks whose rays are dealt to several waves anyhow are not worth a trial
+    if (g_task_split == 2 && tasks_are_dealt(s.scene, U)) rec = plan = false;
     if (rec) {
       const uint32_t* before = e.d_split;
       ensure_device(&e.d_split, &e.d_split_cap, (size_t)split_buffer_words(tasks));

@@ -116,6 +116,8 @@ constexpr uint64_t kMaxLaunchUnits = 0xffffffffull - 65536ull;
 // Largest grab of the unit renderer: lane g of a wave holds unit g's count.
 constexpr int kMaxUnitsPerGrab = 64;
 
+// Whether a split launch of U deals each task's rays to several waves.
+bool tasks_are_dealt(const DeviceScene& scene, const UnitLaunch& U);
 // Launches the unit renderer with U's launch shape.
 bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U, hipStream_t stream, std::string* err);
 

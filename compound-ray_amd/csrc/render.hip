@@ -531,6 +531,7 @@ struct RenderArgs {
   // split launches: chunks per unit and the reciprocal of split_unit, tasks, 1 / spp
   uint32_t chunks, chunk_magic, tasks;
   float inv;
+  uint32_t ways_log;   // packet tasks: log2 of the waves a task's rays are dealt to
 };
 typedef __attribute__((address_space(4))) const RenderArgs KernelArgs;
 
@@ -867,6 +868,18 @@ __global__ __launch_bounds__(kTraceThreads, 5) void k_render_chunks(RenderArgs A
   put_partial(fresh_args(), t, lane, r, g, b);
 }
 
+// Which of 2^ways_log waves traces a sample: by its azimuth about the axis (the
+// sign of the splay, then the spin), so that a wave's rays share a sector of
+// the cone; by lane when no more than a ray is left for each (count_log: bits
+// of the task's ray count).
+__device__ __forceinline__ uint32_t cone_sector(const U4& rnd, uint32_t ways_log, uint32_t count_log, int lane) {
+  if (ways_log == 0u) return 0u;
+  if (ways_log + 1u >= count_log) return (uint32_t)lane & ((1u << ways_log) - 1u);
+  // a Box-Muller cosine is negative in the second and third quarter turn
+  const uint32_t back = ((rnd.b >> 30) + 1u) >> 1 & 1u;
+  return ways_log == 1u ? back : back << (ways_log - 1u) | rnd.c >> (33u - ways_log);
+}
+
 // The rays of a task as one packet, in workgroups of one wave.  kSplit: the
 // launch records its tasks' packet steps and, with a list from the last
 // launch's (split_flag), traces the listed tasks first, as several packets.
@@ -907,7 +920,7 @@ __global__ __launch_bounds__(64, 6) void k_render_tasks(RenderArgs A) {
     if (k >= listed) return;  // whole wave
     t = (uint32_t)__builtin_amdgcn_readfirstlane((int)A.U.split_list[first + k]);
   } else {
-    t = wv - sub_waves;
+    t = (wv - sub_waves) >> A.ways_log;
     if (t >= A.tasks) return;  // whole wave
     if (split && __builtin_amdgcn_readfirstlane((int)A.U.split_flag[t]) != 0) return;  // traced listed
   }
@@ -917,9 +930,11 @@ __global__ __launch_bounds__(64, 6) void k_render_tasks(RenderArgs A) {
   const uint32_t s = j * 64u + (uint32_t)lane;
   const bool active = s < (uint32_t)A.U.spp;
   Ray ray;
+  uint32_t sector = 0;
   if (active) {
     const U4 rnd = sample_randoms(A.U.seed, A.U.eye, i, A.U.sample_base + s, A.U.frame, A.U.pose_base);
     ray = generate_ray(A.U.cones[i], A.pose, rnd);
+    sector = cone_sector(rnd, A.ways_log, 32 - __builtin_clz(min(64u, (uint32_t)A.U.spp) | 1u), lane);
   } else {
     ray.ox = ray.oy = ray.oz = 0.0f;
     ray.dx = ray.dy = 0.0f;
@@ -931,6 +946,11 @@ __global__ __launch_bounds__(64, 6) void k_render_tasks(RenderArgs A) {
   // (part + 1) * 64 / ways - 1 by elevation (the direction's y, ties by
   // lane): rays of neighbouring elevation fan out less than the whole chunk.
   bool mine = active;
+  const bool dealt = !kSplit && A.ways_log != 0u;
+  if (dealt) {
+    mine = active && sector == (wv & ((1u << A.ways_log) - 1u));
+    if (__ballot(mine) == 0ull) return;
+  }
   if (part >= 0) {
     const uint32_t bits = __float_as_uint(ray.dy);
     const uint32_t key = ((bits & 0x80000000u) ? ~bits : (bits | 0x80000000u)) & ~63u;
@@ -960,7 +980,7 @@ __global__ __launch_bounds__(64, 6) void k_render_tasks(RenderArgs A) {
     if (kSamples)
       K->U.samples[K->U.sample_offsets[i] + s] = make_float4(c.x, c.y, c.z, h.id != 0xffffffffu ? h.t : -1.0f);
   }
-  if (!kSplit && K->chunks == 1u) {
+  if (!kSplit && K->chunks == 1u && !dealt) {
     // the unit's only chunk
     r = segment_sum(0.0f + r, 64);
     g = segment_sum(0.0f + g, 64);
@@ -970,7 +990,7 @@ __global__ __launch_bounds__(64, 6) void k_render_tasks(RenderArgs A) {
   }
   // a split packet writes its own lanes' terms; the other packets of its
   // task write the rest
-  if (part < 0 || mine) put_partial(K, t, lane, r, g, b);
+  if ((part < 0 && !dealt) || mine) put_partial(K, t, lane, r, g, b);
 }
 
 // Failure-handling probe of the packet traversal's partial-wave guard: one
@@ -1170,6 +1190,27 @@ __global__ __launch_bounds__(kTraceThreads) void k_camera_frame(SceneView S, Cam
   frame[p] = make_color(make_float4(c.x, c.y, c.z, 0.0f));
 }
 
+// A tile of 2^wide_log x 2^high_log pixels, at most 64, per one-wave workgroup,
+// its rays as one packet (641 x 361 pixels of a panorama over 2.2 M triangles:
+// 367 us with a ray per lane and a tree of four children, 136 with tiles of
+// four pixels).
+__global__ __launch_bounds__(64, 6) void k_camera_tiles(SceneView S, CameraLaunch C, int tiles_x, int wide_log,
+                                                        int high_log, uchar4* __restrict__ frame) {
+  extern __shared__ uint32_t tile_lds[];
+  const int lane = (int)(threadIdx.x & 63);
+  const uint32_t tile = xcd_run_block(blockIdx.x, gridDim.x, 16u);
+  const int x = ((int)(tile % (uint32_t)tiles_x) << wide_log) + (lane & ((1 << wide_log) - 1));
+  const int y = ((int)(tile / (uint32_t)tiles_x) << high_log) + (lane >> wide_log);
+  const bool inside = (lane >> wide_log >> high_log) == 0 && x < C.width && y < C.height;
+  const Ray r = camera_ray(C, inside ? x : 0, inside ? y : 0);
+  Hit h;
+  uint32_t steps = 0, tris = 0;
+  packet_hits<kUnitPacketWide>(S, r, precompute_ray(r), inside, tile_lds, h, steps, tris);
+  if (!inside) return;
+  const V3 c = shade(S, h, r.dx, r.dy, r.dz);
+  frame[(size_t)y * C.width + x] = make_color(make_float4(c.x, c.y, c.z, 0.0f));
+}
+
 __global__ void k_frame_sdf(const float4* __restrict__ colours, int omm_count, uchar4* __restrict__ frame,
                             int width) {
   const int x = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1291,6 +1332,38 @@ int render_units_capacity(const DeviceScene& scene, const UnitLaunch& U_in) {
 
 static uint32_t magic_of(int n) { return (uint32_t)std::min<uint64_t>(0xffffffffull, (1ull << 32) / (uint64_t)n); }
 
+// A launch of few packets lasts as long as its longest ones: a wave walks up
+// to 1,500 boxes and 500 triangles of a large scene for 64 rays that fan out
+// (over 60,000 instructions, 100 us and more alone), while most SIMDs have run
+// dry.  Such launches deal their rays to more and narrower packets, up to
+// these many.  Every further packet costs its own ray generation, set-up and
+// walk to its rays, which the short walks of a small scene repay sooner.
+// Measured, us, by packets (rays each):
+//   frames, 24,200 triangles: 1,000 x 100 samples 2k 76, 4k 63, 8k 65, 16k 71,
+//     32k 91; 1,000 x 400 7k 85, 14k 82, 28k 100;
+//   frames, 2.2 M triangles: 700 x 32 700 122, 11k 45, 22k 41; 2,000 x 64 2k
+//     191, 16k 80, 32k 76, 64k 99; 5,500 x 128 11k 242, 22k 169, 44k 150, 88k
+//     188; 5,500 x 500 44k 325, 88k 328;
+//   cameras, 19,602 triangles: 641 x 361 3.6k 97, 7.2k 74, 14k 66, 29k 63, 58k
+//     95; 1,280 x 720 14k 81, 29k 77, 58k 96;
+//   cameras, 2.2 M triangles: 97 x 61 91 722, 5.9k (1) 36; 641 x 361 3.6k 366,
+//     14k 167, 29k 144, 58k 136, 116k 237; 1,280 x 720 14k 312, 58k 202, 115k
+//     254; 320 x 180 29k (2) 80, 58k (1) 123.
+constexpr int kLargeScene = 1 << 18;   // triangles; between the measured sizes
+static uint64_t task_packets(const DeviceScene& scene) { return scene.tri_count < kLargeScene ? 12288 : 49152; }
+static uint64_t tile_packets(const DeviceScene& scene) { return scene.tri_count < kLargeScene ? 16384 : 65536; }
+
+// log2 of the waves that each task of a split launch deals its rays to.
+static int task_ways(const DeviceScene& scene, const UnitLaunch& U) {
+  if (effective_traversal(scene, U.traversal) != kUnitPacketWide) return 0;
+  const uint64_t chunks = U.spp > 64 ? ((uint64_t)U.spp + 63u) / 64u : 1u;
+  const uint64_t tasks = (uint64_t)U.omm_count * chunks, most = task_packets(scene);
+  int ways = 0;
+  while ((std::min(U.spp, 64) >> ways) > 1 && (tasks << (ways + 1)) <= most) ++ways;
+  return ways;
+}
+bool tasks_are_dealt(const DeviceScene& scene, const UnitLaunch& U) { return task_ways(scene, U) > 0; }
+
 bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipStream_t stream, std::string* err) {
   UnitLaunch U = U_in;
   const uint64_t units = (uint64_t)U.pose_count * (uint64_t)U.omm_count;
@@ -1369,7 +1442,9 @@ bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipSt
                            : (wide ? k_render_tasks<false, kW, true> : k_render_tasks<false, kP, true>);
         reduce = true;
       }
-      const uint64_t waves = tasks + (A.U.split_flag ? (uint64_t)kSplitSubWaves : 0u);
+      if (!A.U.split_cost) A.ways_log = (uint32_t)task_ways(scene, U);
+      if (A.ways_log != 0u) reduce = true;
+      const uint64_t waves = (tasks << A.ways_log) + (A.U.split_flag ? (uint64_t)kSplitSubWaves : 0u);
       hipLaunchKernelGGL(kernel, dim3((unsigned)waves), dim3(64), units_lds_bytes(scene, U.traversal, 1), stream, A);
       g_last_kernel = "k_render_tasks";
     } else {
@@ -1392,11 +1467,15 @@ bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipSt
     return check_launch("render_tasks", err);
   }
   // Units per wave: as given, or (0) as many as leave four waves for every
-  // resident slot, at most auto_grab_max, but enough to fill a wave's lanes.
+  // resident slot, at most auto_grab_max, but enough to fill a wave's lanes
+  // where that does not leave too few packets (733 ommatidia x 15 samples x 17
+  // poses: 3,115 waves of four units 183 us with all else, 12,461 of one 115).
   if (A.U.units_per_grab <= 0) {
     uint64_t fill = 1;
+    const uint64_t few = U.traversal == kUnitPacketWide ? task_packets(scene) : 0;
     if (one_pass(U))
-      for (uint64_t seg = 64; seg > 1 && seg / 2 >= (uint64_t)std::max(U.spp, 1); seg /= 2) fill *= 2;
+      for (uint64_t seg = 64; seg > 1 && seg / 2 >= (uint64_t)std::max(U.spp, 1) && units / (2 * fill) >= few; seg /= 2)
+        fill *= 2;
     A.U.units_per_grab = (int)std::max<uint64_t>(
         fill, std::min<uint64_t>((uint64_t)std::max(U.auto_grab_max, 1), units / (4 * resident_waves)));
   }
@@ -1482,6 +1561,20 @@ bool launch_camera_frame(const DeviceScene& scene, const CameraLaunch& C, uchar4
   if (pixels > 0x7fffffffLL) {
     if (err) *err = "camera: frame too large";
     return false;
+  }
+  if (frame && !rays && scene.node_count > 0 && effective_traversal(scene, kUnitPacketWide) == kUnitPacketWide) {
+    // the smallest tile (1, 1 x 2, 2 x 2 .. 8 x 8 pixels) that makes no more
+    // than tile_packets tiles; single rays are worth a wave only while few
+    int log = 0;
+    if (pixels > 16384) log = 1;
+    while (log < 6 && pixels > (long long)(tile_packets(scene) << log)) ++log;
+    const int wide_log = log / 2, high_log = log - wide_log;
+    const int tiles_x = (C.width + (1 << wide_log) - 1) >> wide_log;
+    const int tiles_y = (C.height + (1 << high_log) - 1) >> high_log;
+    hipLaunchKernelGGL(k_camera_tiles, dim3((unsigned)(tiles_x * tiles_y)), dim3(64),
+                       units_lds_bytes(scene, kUnitPacketWide, 1), stream, view_of(scene), C, tiles_x, wide_log,
+                       high_log, frame);
+    return check_launch("camera_frame", err);
   }
   const size_t lds = stack_bytes(scene);
   if (lds > 160 * 1024) {
