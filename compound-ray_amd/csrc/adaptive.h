@@ -84,7 +84,8 @@ class AdaptiveRenderer {
   size_t poses_cap_ = 0;
   float4* d_col_a_ = nullptr;     // pilot colours
   float4* d_col_b_ = nullptr;     // top-up colours
-  float4* d_final_ = nullptr;     // combined colours
+  float* d_final_ = nullptr;      // combined colours, 3 floats each
+  hipStream_t copies_ = nullptr;  // readback beside the render
   float4* d_stats_ = nullptr;     // pilot statistics (2 per unit)
   float* d_feat_ = nullptr;       // kMlpIn per unit
   float* d_pred_ = nullptr;       // per unit

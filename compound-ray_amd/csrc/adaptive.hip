@@ -147,20 +147,23 @@ __global__ __launch_bounds__(kThreads) void k_allocate(const float* __restrict__
 
 // Final colour of each unit into `out`: the pilot mean alone, or pilot and
 // top-up means weighted by their sample counts (the top-up buffer is kept).
+// The final colours, packed as the caller takes them (a float4 copy, read back
+// and repacked by the host, took 2-3 ms of a render of a million units).
 __global__ void k_combine(const float4* __restrict__ a, const float4* __restrict__ b,
-                          const uint32_t* __restrict__ extra, int pilot, uint64_t units, float4* __restrict__ out) {
+                          const uint32_t* __restrict__ extra, int pilot, uint64_t units, float* __restrict__ out) {
   const uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (u >= units) return;
   const float4 ca = a[u];
   const uint32_t e = extra[u];
-  if (e == 0) {
-    out[u] = make_float4(ca.x, ca.y, ca.z, (float)pilot);
-    return;
+  V3 c = v3(ca.x, ca.y, ca.z);
+  if (e != 0) {
+    const float4 cb = b[u];
+    const float wa = (float)pilot, wb = (float)e, inv = 1.0f / (wa + wb);
+    c = v3((wa * ca.x + wb * cb.x) * inv, (wa * ca.y + wb * cb.y) * inv, (wa * ca.z + wb * cb.z) * inv);
   }
-  const float4 cb = b[u];
-  const float wa = (float)pilot, wb = (float)e, inv = 1.0f / (wa + wb);
-  out[u] = make_float4((wa * ca.x + wb * cb.x) * inv, (wa * ca.y + wb * cb.y) * inv, (wa * ca.z + wb * cb.z) * inv,
-                       wa + wb);
+  out[3 * u] = c.x;
+  out[3 * u + 1] = c.y;
+  out[3 * u + 2] = c.z;
 }
 // Training labels from a long render's statistics: log2(max(n_req, 1)), n_req
 // = mean RGB variance / error^2, clamped to [0, 12].
@@ -220,14 +223,16 @@ void AdaptiveRenderer::release() {
   d_poses_ = nullptr;
   d_part_ = d_sqrt_ = nullptr;
   part_cap_ = 0;
-  d_col_a_ = d_col_b_ = d_final_ = d_stats_ = nullptr;
-  d_feat_ = d_pred_ = nullptr;
+  d_col_a_ = d_col_b_ = d_stats_ = nullptr;
+  d_feat_ = d_pred_ = d_final_ = nullptr;
   d_counts_ = d_extra_ = nullptr;
   d_total_ = nullptr;
   poses_cap_ = units_cap_ = 0;
   if (ev0_) (void)hipEventDestroy(ev0_);
   if (ev1_) (void)hipEventDestroy(ev1_);
   ev0_ = ev1_ = nullptr;
+  if (copies_) (void)hipStreamDestroy(copies_);
+  copies_ = nullptr;
   for (hipEvent_t& e : ev_stage_) {
     if (e) (void)hipEventDestroy(e);
     e = nullptr;
@@ -239,6 +244,10 @@ bool AdaptiveRenderer::ensure(size_t poses, size_t units, std::string* err) {
                 hipEventCreate(&ev_stage_[0]) != hipSuccess || hipEventCreate(&ev_stage_[1]) != hipSuccess ||
                 hipEventCreate(&ev_stage_[2]) != hipSuccess)) {
     if (err) *err = "adaptive: event creation failed";
+    return false;
+  }
+  if (!copies_ && hipStreamCreateWithFlags(&copies_, hipStreamNonBlocking) != hipSuccess) {
+    if (err) *err = "adaptive: stream creation failed";
     return false;
   }
   if (!d_total_ && !grow(&d_total_, 1, err)) return false;
@@ -253,7 +262,7 @@ bool AdaptiveRenderer::ensure(size_t poses, size_t units, std::string* err) {
     part_cap_ = parts;
   }
   if (units > units_cap_) {
-    if (!grow(&d_col_a_, units, err) || !grow(&d_col_b_, units, err) || !grow(&d_final_, units, err) ||
+    if (!grow(&d_col_a_, units, err) || !grow(&d_col_b_, units, err) || !grow(&d_final_, 3 * units, err) ||
         !grow(&d_stats_, 2 * units, err) ||
         !grow(&d_feat_, units * kMlpIn, err) || !grow(&d_pred_, units, err) || !grow(&d_counts_, units, err) ||
         !grow(&d_extra_, units, err))
@@ -348,6 +357,16 @@ bool AdaptiveRenderer::render(const DeviceScene& scene, UnitLaunch U, const std:
                      (uint64_t)units, d_final_);
   if (!ok_launch("combine", err)) return false;
   (void)hipEventRecord(ev1_, stream);
+  // the counts are final since the allocation: they cross to the host while
+  // the top-up renders
+  if (counts && (hipStreamWaitEvent(copies_, ev_stage_[1], 0) != hipSuccess ||
+                 hipMemcpyAsync(counts, d_counts_, sizeof(uint32_t) * units, hipMemcpyDeviceToHost, copies_) !=
+                     hipSuccess ||
+                 hipStreamSynchronize(copies_) != hipSuccess)) {
+    (void)hipStreamSynchronize(stream);
+    if (err) *err = "adaptive: readback failed";
+    return false;
+  }
   unsigned long long total = 0;
   if (hipMemcpyAsync(&total, d_total_, sizeof(total), hipMemcpyDeviceToHost, stream) != hipSuccess ||
       hipStreamSynchronize(stream) != hipSuccess) {
@@ -366,19 +385,7 @@ bool AdaptiveRenderer::render(const DeviceScene& scene, UnitLaunch U, const std:
       res->stage_ms[k] = f;
     }
   }
-  if (rgb) {
-    std::vector<float4> tmp(units);
-    if (hipMemcpy(tmp.data(), d_final_, sizeof(float4) * units, hipMemcpyDeviceToHost) != hipSuccess) {
-      if (err) *err = "adaptive: readback failed";
-      return false;
-    }
-    for (size_t u = 0; u < units; ++u) {
-      rgb[3 * u] = tmp[u].x;
-      rgb[3 * u + 1] = tmp[u].y;
-      rgb[3 * u + 2] = tmp[u].z;
-    }
-  }
-  if (counts && hipMemcpy(counts, d_counts_, sizeof(uint32_t) * units, hipMemcpyDeviceToHost) != hipSuccess) {
+  if (rgb && hipMemcpy(rgb, d_final_, sizeof(float) * 3 * units, hipMemcpyDeviceToHost) != hipSuccess) {
     if (err) *err = "adaptive: readback failed";
     return false;
   }

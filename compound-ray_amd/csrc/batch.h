@@ -68,11 +68,15 @@ class BatchRenderer {
   void release();
 
  private:
+  bool host_rgb();
   bool prepare(const UnitLaunch& U, const std::vector<Pose>& poses, hipStream_t stream, std::string* err);
   Pose* d_poses_ = nullptr;
   size_t poses_cap_ = 0;
   float4* d_colours_ = nullptr;
   size_t colours_cap_ = 0;
+  float* d_rgb_ = nullptr;       // packed for the readback
+  size_t rgb_cap_ = 0;
+  float* h_rgb_ = nullptr;       // the same of small batches, pinned
   hipEvent_t ev0_ = nullptr, ev1_ = nullptr;
 };
 

@@ -58,6 +58,13 @@ struct EyeState {
   float4* d_samples = nullptr;
   size_t d_samples_cap = 0;
   float4* d_colours = nullptr;
+  // Host copy of an eye's colours and pixels that frame kernels write beside
+  // the device's (a blocking copy of each costs 10-15 us, a third of a small
+  // frame): pinned, for eyes of up to kHostColours ommatidia.
+  float4* h_colours = nullptr;
+  uchar4* h_pixels = nullptr;
+  size_t h_cap = 0;
+  size_t h_valid = 0;                    // ommatidia whose last colours it holds
   size_t d_colours_cap = 0;
   bool has_render = false;
   uint64_t rendered_rays = 0;
@@ -108,6 +115,47 @@ struct Cam {
   float start_radius = 0.0f;   // panoramic (PanoramicCamera.cpp:16)
 };
 
+// Buffers of traceRays: two pieces of up to kPiece rays, 48 bytes each.
+struct RayPieces {
+  static constexpr size_t kPiece = 131072;
+  Ray* d_rays[2] = {nullptr, nullptr};
+  int32_t* d_hit[2] = {nullptr, nullptr};
+  float* d_tbb[2] = {nullptr, nullptr};
+  hipStream_t stream[2] = {nullptr, nullptr};
+  size_t rays = 0;   // per piece
+
+  void release() {
+    for (int b = 0; b < 2; ++b) {
+      if (d_rays[b]) (void)hipFree(d_rays[b]);
+      if (d_hit[b]) (void)hipFree(d_hit[b]);
+      if (d_tbb[b]) (void)hipFree(d_tbb[b]);
+      if (stream[b]) (void)hipStreamDestroy(stream[b]);
+      d_rays[b] = nullptr;
+      d_hit[b] = nullptr;
+      d_tbb[b] = nullptr;
+      stream[b] = nullptr;
+    }
+    rays = 0;
+  }
+  void ensure(size_t count) {
+    const size_t n = std::min(count, kPiece);
+    if (rays >= n) return;
+    release();
+    hipError_t e = hipSuccess;
+    for (int b = 0; b < 2; ++b) {
+      if (e == hipSuccess) e = hipMalloc(&d_rays[b], sizeof(Ray) * n);
+      if (e == hipSuccess) e = hipMalloc(&d_hit[b], sizeof(int32_t) * n);
+      if (e == hipSuccess) e = hipMalloc(&d_tbb[b], sizeof(float) * 3 * n);
+      if (e == hipSuccess) e = hipStreamCreateWithFlags(&stream[b], hipStreamNonBlocking);
+    }
+    if (e != hipSuccess) {
+      release();
+      throw std::runtime_error(std::string("traceRays: ") + hipGetErrorString(e));
+    }
+    rays = n;
+  }
+};
+
 struct State {
   bool verbose = true;
   std::string last_error;
@@ -129,6 +177,7 @@ struct State {
   uchar4* d_frame = nullptr;
   size_t d_frame_cap = 0;
   bool frame_host_stale = false;
+  RayPieces rays;
   Pose* d_pose = nullptr;
   uint32_t seed = 42;
   int leaf_max = 4;
@@ -217,6 +266,25 @@ void ensure_device(T** p, size_t* cap, size_t n) {
   *cap = n;
 }
 
+constexpr size_t kHostColours = 65536;
+
+void ensure_host_colours(EyeState& e) {
+  const size_t n = e.omms.size();
+  if (n > kHostColours || (e.h_colours && e.h_cap >= n)) return;
+  if (e.h_colours) (void)hipHostFree(e.h_colours);
+  e.h_colours = nullptr;
+  e.h_cap = e.h_valid = 0;
+  void* p = nullptr;
+  if (n == 0 || hipHostMalloc(&p, n * (sizeof(float4) + sizeof(uchar4)), hipHostMallocMapped | hipHostMallocCoherent) !=
+                    hipSuccess) {
+    (void)hipGetLastError();
+    return;   // frames are read back by copies
+  }
+  e.h_colours = static_cast<float4*>(p);
+  e.h_pixels = reinterpret_cast<uchar4*>(e.h_colours + n);
+  e.h_cap = n;
+}
+
 Cam* current_cam() {
   State& s = st();
   if (s.cams.empty()) return nullptr;
@@ -247,6 +315,7 @@ void free_scene() {
     if (e.d_offsets) (void)hipFree(e.d_offsets);
     if (e.d_samples) (void)hipFree(e.d_samples);
     if (e.d_colours) (void)hipFree(e.d_colours);
+    if (e.h_colours) (void)hipHostFree(e.h_colours);
     if (e.d_proj_ids) (void)hipFree(e.d_proj_ids);
     if (e.d_chunk_partial) (void)hipFree(e.d_chunk_partial);
     if (e.d_split) (void)hipFree(e.d_split);
@@ -438,6 +507,7 @@ void ensure_frame_buffer() {
   if (s.d_frame_cap < n || !s.d_frame) {
     ensure_device(&s.d_frame, &s.d_frame_cap, n);
     if (n) hip_check(hipMemsetAsync(s.d_frame, 0, sizeof(uchar4) * n, s.stream), "clear frame");
+    s.frame_host_stale = true;
   }
 }
 
@@ -467,13 +537,23 @@ double render_compound(EyeState& e, const Cam& c) {
   ensure_device(&e.d_colours, &e.d_colours_cap, e.omms.size());
   ensure_frame_buffer();
   const int omm_count = (int)e.omms.size();
+  ensure_host_colours(e);
+  // whether the host's frame is the device's, so that the pixels of this
+  // render's row are all that it lacks
+  const bool host_frame = !s.frame_host_stale && s.frame_host.size() == 4 * (size_t)s.width * (size_t)s.height;
+  e.h_valid = 0;
   std::string err;
   const auto t0 = std::chrono::steady_clock::now();
   hip_check(hipEventRecord(s.ev[0], s.stream), "event");
   UnitLaunch U = unit_launch_of(e, nullptr, 1);
   U.host_pose = &c.pose;
   U.traced = s.ev[1];
-  bool frame_done = false;
+  bool frame_done = false, host_done = false;
+  if (e.h_colours && e.h_cap >= e.omms.size()) {
+    U.host_colours = e.h_colours;
+    U.host_pixels = e.h_pixels;
+    U.host_done = &host_done;
+  }
   if (e.shader != "single_dimension" && e.shader != "raw_ommatidial_samples" &&
       e.shader.compare(0, 10, "spherical_") != 0) {
     U.frame_pixels = s.d_frame;   // single_dimension_fast
@@ -571,7 +651,11 @@ double render_compound(EyeState& e, const Cam& c) {
   e.frame += 1;
   e.has_render = true;
   e.rendered_rays = record ? total : 0;
-  s.frame_host_stale = true;
+  if (host_done) e.h_valid = e.omms.size();
+  if (host_done && frame_done && host_frame)
+    memcpy(s.frame_host.data(), e.h_pixels, 4 * std::min(e.omms.size(), (size_t)std::max(U.frame_width, 0)));
+  else
+    s.frame_host_stale = true;
   return ms;
 }
 
@@ -771,6 +855,7 @@ void stop(void) {
     (void)hipStreamSynchronize(s.stream);
     free_scene();
     s.batch.release();
+    s.rays.release();
     if (s.d_frame) (void)hipFree(s.d_frame);
     s.d_frame = nullptr;
     s.d_frame_cap = 0;
@@ -1064,12 +1149,17 @@ size_t getOmmatidialColours(float* rgb, size_t count) {
   EyeState* e = current_eye();
   if (!e || !e->has_render || !rgb) return 0;
   const size_t n = std::min(count, e->omms.size());
-  std::vector<float4> tmp(n);
-  if (n) hip_check(hipMemcpy(tmp.data(), e->d_colours, sizeof(float4) * n, hipMemcpyDeviceToHost), "readback");
+  std::vector<float4> tmp;
+  const float4* src = e->h_colours;
+  if (n > e->h_valid) {
+    tmp.resize(n);
+    hip_check(hipMemcpy(tmp.data(), e->d_colours, sizeof(float4) * n, hipMemcpyDeviceToHost), "readback");
+    src = tmp.data();
+  }
   for (size_t i = 0; i < n; ++i) {
-    rgb[3 * i] = tmp[i].x;
-    rgb[3 * i + 1] = tmp[i].y;
-    rgb[3 * i + 2] = tmp[i].z;
+    rgb[3 * i] = src[i].x;
+    rgb[3 * i + 1] = src[i].y;
+    rgb[3 * i + 2] = src[i].z;
   }
   return n;
   ABI_GUARD_END(return 0)
@@ -1226,34 +1316,37 @@ int traceRays(const float* rays, size_t count, int32_t* primIds, float* tbb) {
   if (!s.loaded) throw std::runtime_error("traceRays: no scene loaded");
   if (count == 0) return 0;
   if (!rays || !primIds || !tbb) throw std::runtime_error("traceRays: null argument");
-  Ray* d_rays = nullptr;
-  int32_t* d_hit = nullptr;
-  float4* d_tbb = nullptr;
-  std::string err;
-  bool ok = false;
-  hipError_t he = hipMalloc(&d_rays, sizeof(Ray) * count);
-  if (he == hipSuccess) he = hipMalloc(&d_hit, sizeof(int32_t) * count);
-  if (he == hipSuccess) he = hipMalloc(&d_tbb, sizeof(float4) * count);
-  if (he == hipSuccess) he = hipMemcpy(d_rays, rays, sizeof(Ray) * count, hipMemcpyHostToDevice);
-  if (he == hipSuccess) {
-    ok = launch_trace_rays(s.scene, d_rays, count, d_hit, d_tbb, s.stream, &err);
-    he = hipStreamSynchronize(s.stream);
-  }
-  std::vector<float4> t4;
-  if (ok && he == hipSuccess) {
-    he = hipMemcpy(primIds, d_hit, sizeof(int32_t) * count, hipMemcpyDeviceToHost);
-    t4.resize(count);
-    if (he == hipSuccess) he = hipMemcpy(t4.data(), d_tbb, sizeof(float4) * count, hipMemcpyDeviceToHost);
-  }
-  (void)hipFree(d_rays);
-  (void)hipFree(d_hit);
-  (void)hipFree(d_tbb);
-  if (!ok && !err.empty()) throw std::runtime_error(err);
-  hip_check(he, "traceRays");
-  for (size_t i = 0; i < count; ++i) {
-    tbb[3 * i] = t4[i].x;
-    tbb[3 * i + 1] = t4[i].y;
-    tbb[3 * i + 2] = t4[i].z;
+  // Two halves of a bounded buffer take the rays in turn, each on a stream of
+  // its own: while one piece is traced the next is uploaded and the last
+  // one's hits are read back.
+  RayPieces& P = s.rays;
+  P.ensure(count);
+  const size_t pieces = (count + P.rays - 1) / P.rays, n = (count + pieces - 1) / pieces;
+  const auto read_back = [&](size_t k) {
+    const int b = (int)(k & 1);
+    const size_t first = k * n, m = std::min(n, count - first);
+    hip_check(hipMemcpyAsync(primIds + first, P.d_hit[b], sizeof(int32_t) * m, hipMemcpyDeviceToHost, P.stream[b]),
+              "traceRays");
+    hip_check(hipMemcpyAsync(tbb + 3 * first, P.d_tbb[b], sizeof(float) * 3 * m, hipMemcpyDeviceToHost, P.stream[b]),
+              "traceRays");
+    hip_check(hipStreamSynchronize(P.stream[b]), "traceRays");
+  };
+  try {
+    hip_check(hipStreamSynchronize(s.stream), "traceRays");   // what was queued before this call
+    for (size_t k = 0; k < pieces; ++k) {
+      const int b = (int)(k & 1);
+      const size_t first = k * n, m = std::min(n, count - first);
+      hip_check(hipMemcpyAsync(P.d_rays[b], rays + 8 * first, sizeof(Ray) * m, hipMemcpyHostToDevice, P.stream[b]),
+                "traceRays");
+      std::string err;
+      if (!launch_trace_rays(s.scene, P.d_rays[b], m, P.d_hit[b], P.d_tbb[b], P.stream[b], &err))
+        throw std::runtime_error(err);
+      if (k > 0) read_back(k - 1);
+    }
+    read_back(pieces - 1);
+  } catch (...) {
+    for (hipStream_t q : P.stream) (void)hipStreamSynchronize(q);
+    throw;
   }
   return 0;
   ABI_GUARD_END(return -1)

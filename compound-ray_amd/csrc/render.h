@@ -78,6 +78,11 @@ struct UnitLaunch {
   uchar4* frame_pixels = nullptr;
   int frame_width = 0;
   bool* frame_done = nullptr;
+  // Optional, split launches only: host memory that receives the colours and,
+  // with frame_pixels, the pixels as well; *host_done tells whether it did.
+  float4* host_colours = nullptr;
+  uchar4* host_pixels = nullptr;
+  bool* host_done = nullptr;
   // Optional: recorded after the tracing kernel.
   hipEvent_t traced = nullptr;
   // Optional long-task split of the packet task kernel (an eye rendered frame
@@ -180,7 +185,10 @@ bool launch_generate_rays(const EyeLaunch& L, Ray* rays, hipStream_t stream, std
 bool launch_packet_guard_probe(const DeviceScene& scene, const Ray* rays, int active_lanes, int32_t* ids,
                                hipStream_t stream, std::string* err);
 
-bool launch_trace_rays(const DeviceScene& scene, const Ray* rays, uint64_t n, int32_t* hit,
-                       float4* tbb, hipStream_t stream, std::string* err);
+// hit[r]: the triangle or -1; tbb: t, b1, b2 of each ray.
+bool launch_trace_rays(const DeviceScene& scene, const Ray* rays, uint64_t n, int32_t* hit, float* tbb,
+                       hipStream_t stream, std::string* err);
+// rgb: n packed colours.
+bool launch_pack_rgb(const float4* colours, uint64_t n, float* rgb, hipStream_t stream, std::string* err);
 
 }  // namespace eye

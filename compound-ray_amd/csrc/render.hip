@@ -791,7 +791,12 @@ __device__ __forceinline__ uchar4 make_color(float4 c) {
 __device__ __forceinline__ void put_unit(KernelArgs* K, uint32_t i, float r, float g, float b) {
   const float4 c = make_float4(r, g, b, (float)(uint32_t)K->U.spp);
   K->U.colours[i] = c;
-  if (K->U.frame_pixels && i < (uint32_t)K->U.frame_width) K->U.frame_pixels[i] = make_color(c);
+  if (K->U.host_colours) K->U.host_colours[i] = c;
+  if (K->U.frame_pixels && i < (uint32_t)K->U.frame_width) {
+    const uchar4 pixel = make_color(c);
+    K->U.frame_pixels[i] = pixel;
+    if (K->U.host_pixels) K->U.host_pixels[i] = pixel;
+  }
 }
 
 constexpr uint32_t kTaskFloats = 3 * 64;   // of `partial`, per task
@@ -1161,7 +1166,7 @@ __global__ void k_generate_rays(EyeLaunch L, uint64_t total, Ray* __restrict__ r
 
 __global__ __launch_bounds__(kTraceThreads) void k_trace_rays(SceneView S, const Ray* __restrict__ rays,
                                                               uint64_t n, int32_t* __restrict__ hit,
-                                                              float4* __restrict__ tbb) {
+                                                              float* __restrict__ tbb) {
   extern __shared__ uint32_t lds_stack[];
   const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= n) return;
@@ -1169,7 +1174,9 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_rays(SceneView S, const
   Hit h;
   closest_hit(S, rp, lds_stack + threadIdx.x, blockDim.x, h);
   hit[r] = h.id == 0xffffffffu ? -1 : (int32_t)h.id;
-  tbb[r] = make_float4(h.t, h.b1, h.b2, 0.0f);
+  tbb[3 * r] = h.t;
+  tbb[3 * r + 1] = h.b1;
+  tbb[3 * r + 2] = h.b2;
 }
 
 // One pixel of a regular camera per thread: primary ray, closest hit
@@ -1242,6 +1249,15 @@ __global__ void k_frame_raw(const float4* __restrict__ samples, const uint32_t* 
   const float4 v = samples[first + (size_t)y];
   const float inv = 1.0f / (float)n;
   frame[(size_t)y * width + x] = make_color(make_float4(v.x * inv, v.y * inv, v.z * inv, 0.0f));
+}
+
+__global__ void k_pack_rgb(const float4* __restrict__ colours, uint64_t n, float* __restrict__ rgb) {
+  const uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (u >= n) return;
+  const float4 c = colours[u];
+  rgb[3 * u] = c.x;
+  rgb[3 * u + 1] = c.y;
+  rgb[3 * u + 2] = c.z;
 }
 
 __global__ void k_copy_probe(const float4* __restrict__ src, float4* __restrict__ dst, size_t n) {
@@ -1464,6 +1480,7 @@ bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipSt
     if (reduce)
       hipLaunchKernelGGL(k_reduce_tasks, dim3((unsigned)((units + 3) / 4)), dim3(kTraceThreads), 0, stream, A);
     if (U.frame_done) *U.frame_done = U.frame_pixels != nullptr;
+    if (U.host_done) *U.host_done = U.host_colours != nullptr;
     return check_launch("render_tasks", err);
   }
   // Units per wave: as given, or (0) as many as leave four waves for every
@@ -1586,6 +1603,12 @@ bool launch_camera_frame(const DeviceScene& scene, const CameraLaunch& C, uchar4
   return check_launch("camera_frame", err);
 }
 
+bool launch_pack_rgb(const float4* colours, uint64_t n, float* rgb, hipStream_t stream, std::string* err) {
+  if (n == 0) return true;
+  hipLaunchKernelGGL(k_pack_rgb, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, colours, n, rgb);
+  return check_launch("pack_rgb", err);
+}
+
 bool launch_cones(const Ommatidium* omms, int omm_count, Cone* cones, hipStream_t stream, std::string* err) {
   if (omm_count <= 0) return true;
   hipLaunchKernelGGL(k_cones, dim3((unsigned)((omm_count + 255) / 256)), dim3(256), 0, stream, omms, omm_count, cones);
@@ -1616,7 +1639,7 @@ bool launch_packet_guard_probe(const DeviceScene& scene, const Ray* rays, int ac
   return check_launch("packet_guard_probe", err);
 }
 
-bool launch_trace_rays(const DeviceScene& scene, const Ray* rays, uint64_t n, int32_t* hit, float4* tbb,
+bool launch_trace_rays(const DeviceScene& scene, const Ray* rays, uint64_t n, int32_t* hit, float* tbb,
                        hipStream_t stream, std::string* err) {
   if (n == 0) return true;
   const size_t lds = stack_bytes(scene);
