@@ -324,7 +324,7 @@ struct WideTree {
 
 __device__ __forceinline__ void closest_hit_wide(const WideTree& T, const Ray& ray, const RayPre& rp, bool active,
                                                  uint2* stack, uint32_t* fault, Hit& h, uint32_t& fetched,
-                                                 uint32_t& tris) {
+                                                 uint32_t& tris, float slope = kPacketSlope) {
   h.t = rp.tmax;
   h.b1 = h.b2 = 0.0f;
   h.k = 0xffffffffu;
@@ -369,8 +369,8 @@ __device__ __forceinline__ void closest_hit_wide(const WideTree& T, const Ray& r
     const float k = dot(d, B.w);
     const float rk = __builtin_amdgcn_rcpf(k);
     float a = dot(d, B.u) * rk, b = dot(d, B.v) * rk;
-    const bool in = ((left >> (threadIdx.x & 63)) & 1ull) != 0ull && k > 0.0f && fabsf(a) < kPacketSlope &&
-                    fabsf(b) < kPacketSlope && fabsf(gap.x) + fabsf(gap.y) + fabsf(gap.z) <= T.spread;
+    const bool in = ((left >> (threadIdx.x & 63)) & 1ull) != 0ull && k > 0.0f && fabsf(a) < slope &&
+                    fabsf(b) < slope && fabsf(gap.x) + fabsf(gap.y) + fabsf(gap.z) <= T.spread;
     left &= ~(__ballot(in) | (1ull << first));
     // lanes of other packets take no hits here: their axes may differ
     r.tmin = in ? rp.tmin : INFINITY;
