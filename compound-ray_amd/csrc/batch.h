@@ -34,7 +34,7 @@ struct TuneTrial {
 //   <key> <units_per_grab> <blocks> <traversal> <ms>
 class LaunchTuner {
  public:
-  // grabs {1,2,4,8,16} x blocks {capacity/2, capacity, 2 capacity} x traversal {packet, packet
+  // grabs {1,2,4,8,16} x blocks {0, capacity, 2 capacity} x traversal {packet, packet
   // on the 64-wide tree, per-ray}; capacity is that of the packet kernel
   static std::vector<LaunchShape> candidates(int capacity);
   static std::string key_of(const DeviceScene& scene, const UnitLaunch& U, uint64_t samples_per_pose);
