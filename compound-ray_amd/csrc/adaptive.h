@@ -67,7 +67,7 @@ class AdaptiveRenderer {
   // gets 3 floats per (pose, ommatidium), counts (nullable) the samples used.
   bool render(const DeviceScene& scene, UnitLaunch U, const std::vector<Pose>& poses, Mlp& mlp,
               const AdaptiveConfig& cfg, float* rgb, uint32_t* counts, AdaptiveResult* res, hipStream_t stream,
-              std::string* err);
+              hipStream_t copies, std::string* err);
   // Training rows: features of `pilot` samples and labels log2(n_req) from
   // `label_spp` further samples of the chosen units (unit_mask[pose][omm] != 0).
   bool training_set(const DeviceScene& scene, UnitLaunch U, const std::vector<Pose>& poses,
@@ -85,7 +85,6 @@ class AdaptiveRenderer {
   float4* d_col_a_ = nullptr;     // pilot colours
   float4* d_col_b_ = nullptr;     // top-up colours
   float* d_final_ = nullptr;      // combined colours, 3 floats each
-  hipStream_t copies_ = nullptr;  // readback beside the render
   float4* d_stats_ = nullptr;     // pilot statistics (2 per unit)
   float* d_feat_ = nullptr;       // kMlpIn per unit
   float* d_pred_ = nullptr;       // per unit

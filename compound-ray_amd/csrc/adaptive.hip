@@ -231,8 +231,6 @@ void AdaptiveRenderer::release() {
   if (ev0_) (void)hipEventDestroy(ev0_);
   if (ev1_) (void)hipEventDestroy(ev1_);
   ev0_ = ev1_ = nullptr;
-  if (copies_) (void)hipStreamDestroy(copies_);
-  copies_ = nullptr;
   for (hipEvent_t& e : ev_stage_) {
     if (e) (void)hipEventDestroy(e);
     e = nullptr;
@@ -244,10 +242,6 @@ bool AdaptiveRenderer::ensure(size_t poses, size_t units, std::string* err) {
                 hipEventCreate(&ev_stage_[0]) != hipSuccess || hipEventCreate(&ev_stage_[1]) != hipSuccess ||
                 hipEventCreate(&ev_stage_[2]) != hipSuccess)) {
     if (err) *err = "adaptive: event creation failed";
-    return false;
-  }
-  if (!copies_ && hipStreamCreateWithFlags(&copies_, hipStreamNonBlocking) != hipSuccess) {
-    if (err) *err = "adaptive: stream creation failed";
     return false;
   }
   if (!d_total_ && !grow(&d_total_, 1, err)) return false;
@@ -274,7 +268,7 @@ bool AdaptiveRenderer::ensure(size_t poses, size_t units, std::string* err) {
 
 bool AdaptiveRenderer::render(const DeviceScene& scene, UnitLaunch U, const std::vector<Pose>& poses, Mlp& mlp,
                               const AdaptiveConfig& cfg, float* rgb, uint32_t* counts, AdaptiveResult* res,
-                              hipStream_t stream, std::string* err) {
+                              hipStream_t stream, hipStream_t copies, std::string* err) {
   const size_t np = poses.size();
   const size_t units = np * (size_t)U.omm_count;
   if (units == 0) return true;
@@ -357,12 +351,12 @@ bool AdaptiveRenderer::render(const DeviceScene& scene, UnitLaunch U, const std:
                      (uint64_t)units, d_final_);
   if (!ok_launch("combine", err)) return false;
   (void)hipEventRecord(ev1_, stream);
-  // the counts are final since the allocation: they cross to the host while
-  // the top-up renders
-  if (counts && (hipStreamWaitEvent(copies_, ev_stage_[1], 0) != hipSuccess ||
-                 hipMemcpyAsync(counts, d_counts_, sizeof(uint32_t) * units, hipMemcpyDeviceToHost, copies_) !=
+  // the counts are final since the allocation: they cross to the host, on a
+  // stream of their own, while the top-up renders
+  if (counts && (hipStreamWaitEvent(copies, ev_stage_[1], 0) != hipSuccess ||
+                 hipMemcpyAsync(counts, d_counts_, sizeof(uint32_t) * units, hipMemcpyDeviceToHost, copies) !=
                      hipSuccess ||
-                 hipStreamSynchronize(copies_) != hipSuccess)) {
+                 hipStreamSynchronize(copies) != hipSuccess)) {
     (void)hipStreamSynchronize(stream);
     if (err) *err = "adaptive: readback failed";
     return false;

@@ -121,7 +121,6 @@ struct RayPieces {
   Ray* d_rays[2] = {nullptr, nullptr};
   int32_t* d_hit[2] = {nullptr, nullptr};
   float* d_tbb[2] = {nullptr, nullptr};
-  hipStream_t stream[2] = {nullptr, nullptr};
   size_t rays = 0;   // per piece
 
   void release() {
@@ -129,11 +128,9 @@ struct RayPieces {
       if (d_rays[b]) (void)hipFree(d_rays[b]);
       if (d_hit[b]) (void)hipFree(d_hit[b]);
       if (d_tbb[b]) (void)hipFree(d_tbb[b]);
-      if (stream[b]) (void)hipStreamDestroy(stream[b]);
       d_rays[b] = nullptr;
       d_hit[b] = nullptr;
       d_tbb[b] = nullptr;
-      stream[b] = nullptr;
     }
     rays = 0;
   }
@@ -146,7 +143,6 @@ struct RayPieces {
       if (e == hipSuccess) e = hipMalloc(&d_rays[b], sizeof(Ray) * n);
       if (e == hipSuccess) e = hipMalloc(&d_hit[b], sizeof(int32_t) * n);
       if (e == hipSuccess) e = hipMalloc(&d_tbb[b], sizeof(float) * 3 * n);
-      if (e == hipSuccess) e = hipStreamCreateWithFlags(&stream[b], hipStreamNonBlocking);
     }
     if (e != hipSuccess) {
       release();
@@ -178,6 +174,9 @@ struct State {
   size_t d_frame_cap = 0;
   bool frame_host_stale = false;
   RayPieces rays;
+  // what runs beside `stream` (one stream for all of it: more streams than
+  // hardware queues share a queue and no longer overlap)
+  hipStream_t side = nullptr;
   Pose* d_pose = nullptr;
   uint32_t seed = 42;
   int leaf_max = 4;
@@ -231,6 +230,7 @@ void ensure_hip() {
   if (e != hipSuccess || count == 0) throw std::runtime_error("no HIP device available");
   hip_check(hipSetDevice(0), "hipSetDevice");
   hip_check(hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking), "hipStreamCreate");
+  hip_check(hipStreamCreateWithFlags(&s.side, hipStreamNonBlocking), "hipStreamCreate");
   hip_check(hipMalloc(&s.d_pose, sizeof(Pose)), "hipMalloc pose");
   hip_check(hipMalloc(&s.d_stats, sizeof(unsigned long long) * 4), "hipMalloc stats");
   hip_check(hipMalloc(&s.d_packet_counts, sizeof(unsigned long long) * 2), "hipMalloc packet counts");
@@ -1322,32 +1322,33 @@ int traceRays(const float* rays, size_t count, int32_t* primIds, float* tbb) {
   // one's hits are read back (300,007 rays in 2.2 M triangles in one piece 1.18
   // ms, in pieces of 65,536 0.97, of 131,072 0.90).
   RayPieces& P = s.rays;
+  const hipStream_t stream[2] = {s.stream, s.side};
   P.ensure(count);
   const size_t pieces = (count + P.rays - 1) / P.rays, n = (count + pieces - 1) / pieces;
   const auto read_back = [&](size_t k) {
     const int b = (int)(k & 1);
     const size_t first = k * n, m = std::min(n, count - first);
-    hip_check(hipMemcpyAsync(primIds + first, P.d_hit[b], sizeof(int32_t) * m, hipMemcpyDeviceToHost, P.stream[b]),
+    hip_check(hipMemcpyAsync(primIds + first, P.d_hit[b], sizeof(int32_t) * m, hipMemcpyDeviceToHost, stream[b]),
               "traceRays");
-    hip_check(hipMemcpyAsync(tbb + 3 * first, P.d_tbb[b], sizeof(float) * 3 * m, hipMemcpyDeviceToHost, P.stream[b]),
+    hip_check(hipMemcpyAsync(tbb + 3 * first, P.d_tbb[b], sizeof(float) * 3 * m, hipMemcpyDeviceToHost, stream[b]),
               "traceRays");
-    hip_check(hipStreamSynchronize(P.stream[b]), "traceRays");
+    hip_check(hipStreamSynchronize(stream[b]), "traceRays");
   };
   try {
     hip_check(hipStreamSynchronize(s.stream), "traceRays");   // what was queued before this call
     for (size_t k = 0; k < pieces; ++k) {
       const int b = (int)(k & 1);
       const size_t first = k * n, m = std::min(n, count - first);
-      hip_check(hipMemcpyAsync(P.d_rays[b], rays + 8 * first, sizeof(Ray) * m, hipMemcpyHostToDevice, P.stream[b]),
+      hip_check(hipMemcpyAsync(P.d_rays[b], rays + 8 * first, sizeof(Ray) * m, hipMemcpyHostToDevice, stream[b]),
                 "traceRays");
       std::string err;
-      if (!launch_trace_rays(s.scene, P.d_rays[b], m, P.d_hit[b], P.d_tbb[b], P.stream[b], &err))
+      if (!launch_trace_rays(s.scene, P.d_rays[b], m, P.d_hit[b], P.d_tbb[b], stream[b], &err))
         throw std::runtime_error(err);
       if (k > 0) read_back(k - 1);
     }
     read_back(pieces - 1);
   } catch (...) {
-    for (hipStream_t q : P.stream) (void)hipStreamSynchronize(q);
+    for (hipStream_t q : stream) (void)hipStreamSynchronize(q);
     throw;
   }
   check_packet_fault("traceRays");
@@ -1689,7 +1690,7 @@ double renderPoseBatchAdaptive(const float* poses, size_t poseCount, float error
   std::string err;
   UnitLaunch U = unit_launch_of(*e, nullptr, (int)poseCount);
   if (!s.adaptive.render(s.scene, U, poses_from6(poses, poseCount), s.mlp, cfg, rgbOut, countsOut, &res, s.stream,
-                         &err))
+                         s.side, &err))
     throw std::runtime_error(err);
   check_packet_fault("renderPoseBatchAdaptive");
   for (int k = 0; k < 4; ++k) s.adaptive_ms[k] = res.stage_ms[k];
