@@ -116,7 +116,7 @@ def cpu_baseline(cfg: dict, spp: int, pose12: np.ndarray, target_s: float = 10.0
 def bench_batched(lib, er, scenes, tmp: str, repeats: int = 3) -> dict:
     """Batched configuration: 4,096 seeded poses of one 5,000-ommatidium eye
     over the 19,602-triangle heightfield, per-ommatidium samples log-uniform in
-    [8, 256], one persistent graph-launched render per batch."""
+    [8, 256], one launch per batch."""
     cfg = scenes.build_config(3, os.path.join(tmp, "c3"))
     lib.loadGlTFscene(str(cfg["gltf"]).encode())
     if er.last_error(lib):
@@ -125,7 +125,7 @@ def bench_batched(lib, er, scenes, tmp: str, repeats: int = 3) -> dict:
     er.set_sample_counts(lib, cfg["counts"])
     poses = cfg["poses"]
     rays = int(cfg["counts"].sum()) * len(poses)
-    # launch shape (units per queue grab, blocks, node-load variant) from the autotuner
+    # launch shape (units per grab, blocks, traversal) from the autotuner
     t0 = time.perf_counter()
     trials = er.autotune_np(lib, poses, repeats=1)
     tune_s = time.perf_counter() - t0
@@ -133,7 +133,7 @@ def bench_batched(lib, er, scenes, tmp: str, repeats: int = 3) -> dict:
     default_ms = float(trials[(trials[:, 0] == 4) & (trials[:, 2] == 0)][:, 3].min())
     log(f"autotune: {len(trials)} shapes in {tune_s:.1f} s -> {tuning}; sample ms best "
         f"{trials[:, 3].min():.2f}, worst {trials[:, 3].max():.2f}")
-    er.render_batch_np(lib, poses, want_rgb=False)  # warm-up (captures the graph)
+    er.render_batch_np(lib, poses, want_rgb=False)  # warm-up
     times = []
     t0 = time.perf_counter()
     for _ in range(repeats):
@@ -781,7 +781,7 @@ def bench_plain(lib, er, cfg: dict, eyes: list, steps: int, warmup: int, trace_m
         "traversal_per_ray": {"nodes": stats["nodes_visited"] / rays_per_step,
                               "tris": stats["tris_tested"] / rays_per_step,
                               "hit_fraction": stats["hits"] / rays_per_step},
-        "roofline": {"bound": "latency of dependent node fetches (L2/MALL-resident scene)",
+        "roofline": {"bound": "VALU issue and the longest packets (L2/MALL-resident scene)",
                      "achieved_packet": packet_launch / (trace_avg_ms * 1e-3) / 1e9,
                      "frac_packet": packet_launch / (trace_avg_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
                      "per_ray_equivalent_GBps": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
@@ -827,7 +827,7 @@ def main() -> int:
     ap.add_argument("--adaptive-only", action="store_true",
                     help="run only learned adaptive sampling at bee scale (profiler runs)")
     ap.add_argument("--batched-only", action="store_true",
-                    help="run only the 4,096-pose batched configuration (profiler runs of the persistent renderer)")
+                    help="run only the 4,096-pose batched configuration (profiler runs)")
     ap.add_argument("--plain-only", action="store_true",
                     help="run only the bee-scale renderFrame workload (profiler runs of k_render_tasks)")
     ap.add_argument("--no-split", action="store_true", help="disable split launches (chunks of a unit on several waves)")

@@ -218,12 +218,15 @@ bool BatchRenderer::render(const DeviceScene& scene, UnitLaunch U, const std::ve
   // pieces of kPackUnits units.  1.1 M units: 1.1 ms less than a float4 copy
   // that the host repacks.
   const bool pinned = rgb && units <= kHostUnits && host_rgb();
+  // without memory to pack into, the host repacks after all
+  std::string no_memory;
+  const bool packs = rgb && (pinned || grow(&d_rgb_, &rgb_cap_, 3 * std::min(kPackUnits, units), &no_memory));
+  if (rgb && !packs) (void)hipGetLastError();
   const auto pack = [&](size_t first) {
-    const size_t n = std::min(kPackUnits, units - first);
-    return (pinned || grow(&d_rgb_, &rgb_cap_, 3 * n, err)) &&
-           launch_pack_rgb(d_colours_ + first, n, pinned ? h_rgb_ : d_rgb_, stream, err);
+    return launch_pack_rgb(d_colours_ + first, std::min(kPackUnits, units - first), pinned ? h_rgb_ : d_rgb_, stream,
+                           err);
   };
-  if (rgb && !pack(0)) {
+  if (packs && !pack(0)) {
     (void)hipStreamSynchronize(stream);
     return false;
   }
@@ -236,6 +239,19 @@ bool BatchRenderer::render(const DeviceScene& scene, UnitLaunch U, const std::ve
   *gpu_ms = ms;
   if (pinned) {
     memcpy(rgb, h_rgb_, sizeof(float) * 3 * units);
+    return true;
+  }
+  if (rgb && !packs) {
+    std::vector<float4> tmp(units);
+    if (hipMemcpy(tmp.data(), d_colours_, sizeof(float4) * units, hipMemcpyDeviceToHost) != hipSuccess) {
+      if (err) *err = "batch: readback failed";
+      return false;
+    }
+    for (size_t i = 0; i < units; ++i) {
+      rgb[3 * i] = tmp[i].x;
+      rgb[3 * i + 1] = tmp[i].y;
+      rgb[3 * i + 2] = tmp[i].z;
+    }
     return true;
   }
   for (size_t first = 0; rgb && first < units; first += kPackUnits) {
