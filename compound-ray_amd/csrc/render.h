@@ -172,20 +172,19 @@ bool launch_frame_raw_samples(const float4* samples, const uint32_t* offsets, in
 bool launch_camera_frame(const DeviceScene& scene, const CameraLaunch& C, uchar4* frame, Ray* rays,
                          hipStream_t stream, std::string* err);
 
-// Rays of one eye at one pose, in (ommatidium, sample) order, 8 floats each.
 // cones[i] = cone_of(omms[i]).
 bool launch_cones(const Ommatidium* omms, int omm_count, Cone* cones, hipStream_t stream, std::string* err);
+// Rays of one eye at one pose, in (ommatidium, sample) order, 8 floats each.
 bool launch_generate_rays(const EyeLaunch& L, Ray* rays, hipStream_t stream, std::string* err);
 
-// Closest hits of arbitrary rays: hit[i] = original triangle id or -1,
-// tbb[i] = (t, b1, b2, 0).
 // One wave traces rays[0..63] with the packet traversal; lanes at or above
 // active_lanes skip the call, so below 64 the traversal's partial-wave guard
 // sets the scene's fault word.  ids[lane]: hit id, -1 miss, -2 skipped.
 bool launch_packet_guard_probe(const DeviceScene& scene, const Ray* rays, int active_lanes, int32_t* ids,
                                hipStream_t stream, std::string* err);
 
-// hit[r]: the triangle or -1; tbb: t, b1, b2 of each ray.
+// Closest hits of arbitrary rays: hit[r] = original triangle id or -1, tbb: t,
+// b1, b2 of each ray.
 bool launch_trace_rays(const DeviceScene& scene, const Ray* rays, uint64_t n, int32_t* hit, float* tbb,
                        hipStream_t stream, std::string* err);
 // rgb: n packed colours.

@@ -1209,7 +1209,8 @@ __global__ __launch_bounds__(64, 6) void k_trace_packets(SceneView S, const Ray*
 
 // One pixel of a regular camera per thread: primary ray, closest hit
 // (per-ray LDS stack), shading or sky, make_color.  rays (nullable) receives
-// the generated rays.
+// the generated rays.  Frames take k_camera_tiles where there is a 64-wide
+// tree.
 __global__ __launch_bounds__(kTraceThreads) void k_camera_frame(SceneView S, CameraLaunch C,
                                                                 uchar4* __restrict__ frame, Ray* __restrict__ rays) {
   extern __shared__ uint32_t lds_stack[];

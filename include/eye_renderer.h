@@ -291,7 +291,8 @@ void setSplitLaunches(bool enabled);
  * whole.  mode 0: never; 1: always;
  * 2 (default): per eye, by the measured trace times of a few renders with and
  * without it, tried again every 1,000 renders and after any change of the
- * rays.  Results are the same either way.  No counterpart in the reference
+ * rays; frames of so few tasks that their rays are dealt to several waves
+ * anyhow are not tried.  Results are the same either way.  No counterpart in the reference
  * (scheduling of this renderer). */
 void setTaskSplit(int mode);
 /* Tasks of the last renderFrame of the current eye traced as several packets
