@@ -83,6 +83,7 @@ __device__ __forceinline__ void wave_max6(float& a, float& b, float& c, float& d
   e = lane_f(e, 63);
   f = lane_f(f, 63);
 }
+// The maximum of a value that is not negative in any lane: compared as bits.
 template <int kCtrl, int kRows = 0xf>
 __device__ __forceinline__ int dpp_i(int i) {
   return __builtin_amdgcn_update_dpp(i, i, kCtrl, kRows, 0xf, false);
@@ -107,7 +108,7 @@ struct PacketBounds {
   float a0, a1, b0, b1;       // slopes
   float oa0, oa1, ob0, ob1;   // plane offsets
   float near;                 // smallest start depth along w
-  float spread;               // largest start depth beyond it
+  float spread;               // largest origin depth beyond it
   float reach;                // largest depth along w per unit of t
   float pad;                  // far origins only: added to half extents
 };
@@ -214,7 +215,7 @@ constexpr uint32_t kWideFetch = sizeof(WideNode64) / 128;
 // lane reads).  stack: the wave's LDS column (wide_stack entries).  fetched /
 // tris count node bytes / 128 and leaf triangles (wave-uniform).  kFar: the
 // origins lie far outside the scene, whose boxes' padding does not cover
-// them.
+// them, or rays start behind theirs and may hit there, at a negative t.
 template <bool kShared, bool kFar>
 __device__ __forceinline__ void walk64(const WideNode64* nodes, const float4* wtris, int root, const PacketBounds& B,
                                        const PacketRay& r, bool in, int axes, uint2* stack, Hit& h,
@@ -222,8 +223,11 @@ __device__ __forceinline__ void walk64(const WideNode64* nodes, const float4* wt
   const int lane = (int)(threadIdx.x & 63);
   int sp = 0;
   int node = root;
-  float limit = in ? h.t * kCullSlack : -INFINITY;
-  float horizon = INFINITY;   // depth beyond which every ray has a closer hit
+  const auto cull_limit = [](float t) { return kFar ? fmaf(fabsf(t), kCullSlack - 1.0f, t) : t * kCullSlack; };
+  float limit = in ? cull_limit(h.t) : -INFINITY;
+  // Depth beyond which every ray has a closer hit: depths count from the
+  // starts, a hit's t from its ray's origin.
+  float horizon = INFINITY;
   for (;;) {
     node = __builtin_amdgcn_readfirstlane(node);
     fetched += kWideFetch;
@@ -255,13 +259,13 @@ __device__ __forceinline__ void walk64(const WideNode64* nodes, const float4* wt
           tris += leaf_count(code);
           const float before = h.t;
           test_leaf64<kShared>(wtris, code, r, axes, h);
-          limit = in ? h.t * kCullSlack : -INFINITY;
+          limit = in ? cull_limit(h.t) : -INFINITY;
           closer = closer || __ballot(h.t < before) != 0ull;
         }
         box = next;
       } while (leaves != 0ull);
     }
-    if (closer) horizon = wave_max_depth(in ? h.t : 0.0f) * B.reach + B.spread;
+    if (closer) horizon = wave_max_depth(in ? (kFar ? fmaxf(h.t, 0.0f) : h.t) : 0.0f) * B.reach + B.spread;
     uint64_t kept = 0ull;
     if (inner != 0ull) {
       int l = __builtin_ctzll(inner);
@@ -311,6 +315,29 @@ __device__ __forceinline__ void walk64(const WideNode64* nodes, const float4* wt
 // cones, or several eyes.
 constexpr float kPacketSlope = 1.0f;
 constexpr float kPacketSpread = 1.0f / 256.0f;
+constexpr float kFarStart = 1e30f;
+
+// The offsets and depths of B for rays that start `back` <= 0 times d behind
+// their origins o, all of them within `out` of 0 along each axis.  From starts
+// so far behind that they cannot be computed with (tmin may be infinite) the
+// packet has no bounds.
+__device__ __forceinline__ void bound_starts_behind(PacketBounds& B, const V3& o, const V3& d, float back, bool in,
+                                                    float out) {
+  const V3 p = v3(fmaf(back, d.x, o.x), fmaf(back, d.y, o.y), fmaf(back, d.z, o.z));
+  const float away = fabsf(p.x) + fabsf(p.y) + fabsf(p.z);
+  const float pu = dot(p, B.u), pv = dot(p, B.v), pw = dot(p, B.w);
+  float oa1 = pu - B.a1 * pw, oa0 = B.a0 * pw - pu, ob1 = pv - B.b1 * pw, ob0 = B.b0 * pw - pv, nr = -pw,
+        fr = dot(o, B.w);
+  wave_max6(oa0, oa1, ob0, ob1, nr, fr);
+  const float m = 8.0f * kWidePad * fmaxf(out, wave_max_depth(in && away < kFarStart ? away : 0.0f));
+  const bool bounded = __ballot(in && !(away < kFarStart)) == 0ull;
+  B.oa0 = first_f(bounded ? oa0 + m : INFINITY);
+  B.oa1 = first_f(bounded ? oa1 + m : INFINITY);
+  B.ob0 = first_f(bounded ? ob0 + m : INFINITY);
+  B.ob1 = first_f(bounded ? ob1 + m : INFINITY);
+  B.near = first_f(bounded ? -nr - m : -INFINITY);
+  B.spread = first_f(bounded ? (fr + nr) + 2.0f * m : INFINITY);
+}
 
 // Closest hits of the wave's rays (ray, rp: this lane's) in the tree of T.
 struct WideTree {
@@ -385,27 +412,29 @@ __device__ __forceinline__ void closest_hit_wide(const WideTree& T, const Ray& r
     B.b1 = first_f(b1 + margin);
     B.reach = reach * 1.0002f;
     B.pad = 2.0f * kWidePad * out;
-    // where the rays start: a negative tmin starts behind the origin
-    const float back = fminf(rp.tmin, 0.0f);
-    const V3 p0 = v3(fmaf(back, ray.dx, ray.ox), fmaf(back, ray.dy, ray.oy), fmaf(back, ray.dz, ray.oz));
-    const V3 p = v3(in ? p0.x : o0.x, in ? p0.y : o0.y, in ? p0.z : o0.z);
-    const float pu = dot(p, B.u), pv = dot(p, B.v), pw = dot(p, B.w);
-    float oa1 = pu - B.a1 * pw, oa0 = B.a0 * pw - pu, ob1 = pv - B.b1 * pw, ob0 = B.b0 * pw - pv, nr = pw, fr = pw;
-    // one start for all rays (samples of one ommatidium): no reductions
-    if (__ballot(p.x != o0.x || p.y != o0.y || p.z != o0.z) != 0ull) {
-      nr = -nr;
-      wave_max6(oa0, oa1, ob0, ob1, nr, fr);
-      nr = -nr;
+    const V3 o = v3(in ? ray.ox : o0.x, in ? ray.oy : o0.y, in ? ray.oz : o0.z);
+    const bool behind = __ballot(in && rp.tmin < 0.0f) != 0ull;
+    if (behind) {
+      bound_starts_behind(B, o, v3(ray.dx, ray.dy, ray.dz), in ? fminf(rp.tmin, 0.0f) : 0.0f, in, out);
+    } else {
+      const float pu = dot(o, B.u), pv = dot(o, B.v), pw = dot(o, B.w);
+      float oa1 = pu - B.a1 * pw, oa0 = B.a0 * pw - pu, ob1 = pv - B.b1 * pw, ob0 = B.b0 * pw - pv, nr = pw, fr = pw;
+      // one start for all rays (samples of one ommatidium): no reductions
+      if (__ballot(o.x != o0.x || o.y != o0.y || o.z != o0.z) != 0ull) {
+        nr = -nr;
+        wave_max6(oa0, oa1, ob0, ob1, nr, fr);
+        nr = -nr;
+      }
+      const float m = 8.0f * kWidePad * out;
+      B.oa0 = first_f(oa0 + m);
+      B.oa1 = first_f(oa1 + m);
+      B.ob0 = first_f(ob0 + m);
+      B.ob1 = first_f(ob1 + m);
+      B.near = first_f(nr - m);
+      B.spread = first_f((fr - nr) + 2.0f * m);
     }
-    const float m = 8.0f * kWidePad * out;
-    B.oa0 = first_f(oa0 + m);
-    B.oa1 = first_f(oa1 + m);
-    B.ob0 = first_f(ob0 + m);
-    B.ob1 = first_f(ob1 + m);
-    B.near = first_f(nr - m);
-    B.spread = first_f((fr - nr) + 2.0f * m);
     const int axes = __builtin_amdgcn_readlane(r.k, first);
-    if (out > T.range)
+    if (behind || out > T.range)
       walk64<false, true>(T.nodes, T.tris, T.root, B, r, in, axes, stack, h, fetched, tris);
     else if (__ballot(in && r.k != axes) == 0ull)
       walk64<true, false>(T.nodes, T.tris, T.root, B, r, in, axes, stack, h, fetched, tris);
