@@ -114,8 +114,7 @@ struct PacketBounds {
 };
 
 // Whether the box may meet the frustum, and its depth beyond the starts along
-// w.  A comparison with a not-a-number (a box with infinite corners) never
-// rejects.
+// w (a number: the boxes are bounded, kWideFarthest).
 __device__ __forceinline__ bool bounds_meet(const PacketBounds& B, const V3& c, const V3& h, float* depth) {
   const float cu = fmaf(c.z, B.u.z, fmaf(c.y, B.u.y, c.x * B.u.x));
   const float cv = fmaf(c.z, B.v.z, fmaf(c.y, B.v.y, c.x * B.v.x));
@@ -142,7 +141,7 @@ struct PacketRay {
 };
 
 // Whether the ray enters the box before `limit`.  The rounding of the test is
-// within the boxes' padding; a not-a-number never rejects.
+// within the boxes' padding.
 __device__ __forceinline__ bool ray_meets(const PacketRay& r, float cx, float cy, float cz, float hx, float hy,
                                           float hz, float limit) {
   const float tx = fmaf(cx, r.ix, r.nx), ty = fmaf(cy, r.iy, r.ny), tz = fmaf(cz, r.iz, r.nz);

@@ -46,6 +46,13 @@ constexpr int kWideStackMax = 512;
 // Relative padding of box tests: eight times the rounding of a test.
 constexpr float kWidePad = 4.76837158203125e-7f;   // 2^-21
 
+// Scenes with a vertex that is not a number or further out than this have no
+// wide tree: boxes as centre and half extent would lose such corners (an
+// infinite or overflowing centre is not inside its box), and a packet orders
+// children by depths, which have to be numbers.  Their rays take the 4-wide
+// walks, whose boxes keep both corners.
+constexpr float kWideFarthest = 1.152921504606846976e18f;   // 2^60
+
 // Boxes as centre and half extent: (c - o) / d -/+ h / |d| needs no choice of
 // near and far planes.  Half extents are rounded up and padded by kWidePad of
 // themselves, of the centre and of the scene's radius R (the largest
@@ -62,7 +69,7 @@ struct alignas(32) WideNode64 {
 static_assert(sizeof(WideNode64) == 2048, "wide node layout");
 
 // Builds scene->wide_* from the scene's canonical triangles; without room for
-// it they stay null.  False and `err` on failure (nothing is left allocated).
+// it, or beyond kWideFarthest, they stay null.  False and `err` on failure (nothing is left allocated).
 bool build_wide_tree(DeviceScene* scene, hipStream_t stream, std::string* err);
 void free_wide_tree(DeviceScene* scene);
 

@@ -30,7 +30,6 @@ __device__ __forceinline__ uint64_t expand_bits21(uint64_t v) {
   return (v | v << 2) & 0x1249249249249249ull;
 }
 
-// Not-a-number coordinates (a triangle no ray can hit) are left out.
 __device__ __forceinline__ void tri_box(const float4* tris, size_t k, float lo[3], float hi[3]) {
   const float4 a = tris[3 * k], b = tris[3 * k + 1], c = tris[3 * k + 2];
   lo[0] = fminf(fminf(a.x, b.x), c.x);
@@ -44,9 +43,14 @@ __device__ __forceinline__ void tri_box(const float4* tris, size_t k, float lo[3
 __global__ __launch_bounds__(kBuildThreads) void k_wide_codes(const float4* __restrict__ tris, int n, float ox,
                                                              float oy, float oz, float scale,
                                                              uint64_t* __restrict__ codes,
-                                                             uint32_t* __restrict__ ids) {
+                                                             uint32_t* __restrict__ ids,
+                                                             uint32_t* __restrict__ beyond) {
   const int i = blockIdx.x * kBuildThreads + threadIdx.x;
   if (i >= n) return;
+  const auto within = [](const float4& v) {   // false for a not-a-number
+    return (fabsf(v.x) <= kWideFarthest) & (fabsf(v.y) <= kWideFarthest) & (fabsf(v.z) <= kWideFarthest);
+  };
+  if (!(within(tris[3 * (size_t)i]) & within(tris[3 * (size_t)i + 1]) & within(tris[3 * (size_t)i + 2]))) *beyond = 1u;
   float lo[3], hi[3];
   tri_box(tris, (size_t)i, lo, hi);
   const float o[3] = {ox, oy, oz};
@@ -322,7 +326,8 @@ bool good(hipError_t e, const char* what, std::string* err) {
   return false;
 }
 
-bool build(DeviceScene* S, Pool& pool, ScanScratch* scan, hipStream_t stream, std::string* err) {
+// *unfit: the scene takes no wide tree.
+bool build(DeviceScene* S, Pool& pool, ScanScratch* scan, bool* unfit, hipStream_t stream, std::string* err) {
   const int n = S->tri_count;
   const size_t N = (size_t)n;
   const int tiles = (int)((N + kSortTile - 1) / kSortTile);
@@ -331,6 +336,7 @@ bool build(DeviceScene* S, Pool& pool, ScanScratch* scan, hipStream_t stream, st
   uint32_t* hist = pool.get<uint32_t>((size_t)kRadix * tiles);
   int2* range = pool.get<int2>(2 * N - 1);
   int32_t* parent = pool.get<int32_t>(2 * N - 1);
+  uint32_t* bad = pool.get<uint32_t>(1);
   if (!pool.ok || !scan_reserve(scan, std::max((size_t)kRadix * tiles, N + 1), err)) return false;
   float ext = 0.0f;
   for (int a = 0; a < 3; ++a) ext = std::max(ext, S->centroid_hi[a] - S->centroid_lo[a]);
@@ -338,8 +344,18 @@ bool build(DeviceScene* S, Pool& pool, ScanScratch* scan, hipStream_t stream, st
   for (int a = 0; a < 3; ++a)
     radius = std::max(radius, std::max(std::fabs(S->centroid_lo[a]), std::fabs(S->centroid_hi[a])));
   const float scale = ext > 0.0f ? 2097152.0f / ext : 0.0f;
+  if (!good(hipMemsetAsync(bad, 0, sizeof(uint32_t), stream), "clear", err)) return false;
   hipLaunchKernelGGL(k_wide_codes, dim3(blocks_of(N)), dim3(kBuildThreads), 0, stream, S->tris, n, S->centroid_lo[0],
-                     S->centroid_lo[1], S->centroid_lo[2], scale, codes, ids);
+                     S->centroid_lo[1], S->centroid_lo[2], scale, codes, ids, bad);
+  uint32_t beyond = 0;
+  if (!good(hipGetLastError(), "launch", err) ||
+      !good(hipMemcpyAsync(&beyond, bad, sizeof(beyond), hipMemcpyDeviceToHost, stream), "extent", err) ||
+      !good(hipStreamSynchronize(stream), "extent", err))
+    return false;
+  if (beyond) {
+    *unfit = true;
+    return true;
+  }
   for (int shift = 0; shift < 64; shift += 8) {
     hipLaunchKernelGGL(k_sort_hist<uint64_t>, dim3(tiles), dim3(kSortThreads), 0, stream, codes, n, shift, hist,
                        tiles);
@@ -412,7 +428,6 @@ bool build(DeviceScene* S, Pool& pool, ScanScratch* scan, hipStream_t stream, st
   WideNode64* nodes = pool.get<WideNode64>((size_t)total);
   float4* tris = pool.get<float4>(3 * N);
   uint32_t* parents = pool.get<uint32_t>((size_t)total);
-  uint32_t* bad = pool.get<uint32_t>(1);
   if (!pool.ok) return false;
   size_t at = 0;
   for (const Level& l : levels) {
@@ -457,7 +472,8 @@ bool build_wide_tree(DeviceScene* scene, hipStream_t stream, std::string* err) {
   ScanScratch scan;
   Pool pool;
   pool.err = err;
-  const bool ok = build(scene, pool, &scan, stream, err);
+  bool unfit = false;
+  const bool ok = build(scene, pool, &scan, &unfit, stream, err);
   scan_release(&scan);
   if (ok || !pool.full) return ok;
   // no room: packets walk the 4-wide tree
