@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstring>
 #include <iostream>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -115,9 +116,11 @@ struct Cam {
   float start_radius = 0.0f;   // panoramic (PanoramicCamera.cpp:16)
 };
 
-// Buffers of traceRays: two pieces of up to kPiece rays, 48 bytes each.
+// Buffers of traceRays: two pieces of up to kPiece rays, 48 bytes each.  A call
+// holds `busy` while it uses them: threads may trace at the same time.
 struct RayPieces {
   static constexpr size_t kPiece = 131072;
+  std::mutex busy;
   Ray* d_rays[2] = {nullptr, nullptr};
   int32_t* d_hit[2] = {nullptr, nullptr};
   float* d_tbb[2] = {nullptr, nullptr};
@@ -856,7 +859,10 @@ void stop(void) {
     (void)hipStreamSynchronize(s.stream);
     free_scene();
     s.batch.release();
-    s.rays.release();
+    {
+      const std::lock_guard<std::mutex> hold(s.rays.busy);
+      s.rays.release();
+    }
     if (s.d_frame) (void)hipFree(s.d_frame);
     s.d_frame = nullptr;
     s.d_frame_cap = 0;
@@ -1322,6 +1328,7 @@ int traceRays(const float* rays, size_t count, int32_t* primIds, float* tbb) {
   // one's hits are read back (300,007 rays in 2.2 M triangles in one piece 1.18
   // ms, in pieces of 65,536 0.97, of 131,072 0.90).
   RayPieces& P = s.rays;
+  const std::lock_guard<std::mutex> hold(P.busy);
   const hipStream_t stream[2] = {s.stream, s.side};
   P.ensure(count);
   const size_t pieces = (count + P.rays - 1) / P.rays, n = (count + pieces - 1) / pieces;
