@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <string>
 
+#include "launch_grid.h"
 #include "packet.h"
 #include "render.h"
 
@@ -1457,7 +1458,7 @@ bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipSt
   const bool packet_tasks = U.traversal != kUnitPerRay;
   const uint64_t tasks = units * chunks;
   if (g_split && U.host_pose && !U.omm_counts && !U.unit_counts && !U.stats && (U.spp > 32 || packet_tasks) &&
-      units < 2 * resident_waves && U.chunk_partial && tasks <= 0x7fffffffull - (uint64_t)kSplitSubWaves &&
+      units < 2 * resident_waves && U.chunk_partial && tasks + (uint64_t)kSplitSubWaves <= max_grid(64) &&
       tasks * kTaskFloats <= U.chunk_partial_cap) {
     A.chunks = (uint32_t)chunks;
     A.chunk_magic = magic_of((int)chunks);
@@ -1527,17 +1528,14 @@ bool launch_render_units(const DeviceScene& scene, const UnitLaunch& U_in, hipSt
   }
   A.U.units_per_grab = std::min(A.U.units_per_grab, kMaxUnitsPerGrab);
   const int threads = unit_threads(U.traversal);
-  const uint64_t per_block = (uint64_t)A.U.units_per_grab * (uint64_t)(threads / 64);
-  A.blocks = (uint32_t)((units + per_block - 1) / per_block);
+  const UnitGrid shape = unit_grid(units, A.U.units_per_grab, threads, U.blocks);
+  A.blocks = shape.blocks;
   // eight runs of consecutive workgroups per XCD: long enough for its L2 to
   // hold a pose's surroundings, short enough to even out the XCDs' work (4 to
   // 16 runs within 1 %, 64 runs 3-10 % slower)
   A.run = std::max<uint32_t>(1u, A.blocks / (kXcds * 8u));
-  const uint32_t grid =
-      U.blocks > 0 ? (uint32_t)std::min<uint64_t>((uint64_t)U.blocks * (uint64_t)(kTraceThreads / threads), A.blocks)
-                   : A.blocks;
-  hipLaunchKernelGGL(units_kernel_of(U), dim3(grid), dim3(threads), units_lds_bytes(scene, U.traversal, threads / 64),
-                     stream, A);
+  hipLaunchKernelGGL(units_kernel_of(U), dim3(shape.grid), dim3(threads),
+                     units_lds_bytes(scene, U.traversal, threads / 64), stream, A);
   if (U.traced) (void)hipEventRecord(U.traced, stream);
   g_last_kernel = "k_render_units";
   return check_launch("render_units", err);
@@ -1608,18 +1606,19 @@ bool launch_camera_frame(const DeviceScene& scene, const CameraLaunch& C, uchar4
     if (err) *err = "camera: frame too large";
     return false;
   }
-  if (frame && !rays && scene.node_count > 0 && effective_traversal(scene, kUnitPacketWide) == kUnitPacketWide) {
-    // the smallest tile (1, 1 x 2, 2 x 2 .. 8 x 8 pixels) that makes no more
-    // than tile_packets tiles; single rays are worth a wave only while few
-    int log = 0;
-    if (pixels > 16384) log = 1;
-    while (log < 6 && pixels > (long long)(tile_packets(scene) << log)) ++log;
-    const int wide_log = log / 2, high_log = log - wide_log;
-    const int tiles_x = (C.width + (1 << wide_log) - 1) >> wide_log;
-    const int tiles_y = (C.height + (1 << high_log) - 1) >> high_log;
+  // the smallest tile (1, 1 x 2, 2 x 2 .. 8 x 8 pixels) that makes no more
+  // than tile_packets tiles; single rays are worth a wave only while few
+  int log = 0;
+  if (pixels > 16384) log = 1;
+  while (log < 6 && pixels > (long long)(tile_packets(scene) << log)) ++log;
+  const int wide_log = log / 2, high_log = log - wide_log;
+  const long long tiles_x = ((long long)C.width + (1 << wide_log) - 1) >> wide_log;
+  const long long tiles_y = ((long long)C.height + (1 << high_log) - 1) >> high_log;
+  if (frame && !rays && scene.node_count > 0 && (uint64_t)(tiles_x * tiles_y) <= max_grid(64) &&
+      effective_traversal(scene, kUnitPacketWide) == kUnitPacketWide) {
     hipLaunchKernelGGL(k_camera_tiles, dim3((unsigned)(tiles_x * tiles_y)), dim3(64),
-                       units_lds_bytes(scene, kUnitPacketWide, 1), stream, view_of(scene), C, tiles_x, wide_log,
-                       high_log, frame);
+                       units_lds_bytes(scene, kUnitPacketWide, 1), stream, view_of(scene), C, (int)tiles_x,
+                       wide_log, high_log, frame);
     return check_launch("camera_frame", err);
   }
   const size_t lds = stack_bytes(scene);
@@ -1671,10 +1670,11 @@ bool launch_packet_guard_probe(const DeviceScene& scene, const Ray* rays, int ac
 bool launch_trace_rays(const DeviceScene& scene, const Ray* rays, uint64_t n, int32_t* hit, float* tbb,
                        hipStream_t stream, std::string* err) {
   if (n == 0) return true;
-  if (scene.node_count > 0 && n <= (1ull << 30) &&
+  const int log = n > 16384 ? 3 : 0;
+  const uint64_t packets = (n + (1u << log) - 1) >> log;
+  if (scene.node_count > 0 && packets <= max_grid(64) &&
       effective_traversal(scene, kUnitPacketWide) == kUnitPacketWide) {
-    const int log = n > 16384 ? 3 : 0;
-    hipLaunchKernelGGL(k_trace_packets, dim3((unsigned)((n + (1u << log) - 1) >> log)), dim3(64),
+    hipLaunchKernelGGL(k_trace_packets, dim3((unsigned)packets), dim3(64),
                        units_lds_bytes(scene, kUnitPacketWide, 1), stream, view_of(scene), rays, n, log, hit, tbb);
     return check_launch("trace_rays", err);
   }
