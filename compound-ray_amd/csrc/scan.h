@@ -16,7 +16,8 @@ struct ScanScratch {
   size_t capacity = 0;         // elements the scratch can scan
 };
 
-bool scan_reserve(ScanScratch* s, size_t n, std::string* err);
+// *full (nullable): whether it failed for want of memory.
+bool scan_reserve(ScanScratch* s, size_t n, std::string* err, bool* full = nullptr);
 void scan_release(ScanScratch* s);
 // In place: data[i] <- sum of data[0..i-1].
 bool scan_exclusive_u32(ScanScratch* s, uint32_t* data, size_t n, hipStream_t stream, std::string* err);

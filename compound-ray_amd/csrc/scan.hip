@@ -74,7 +74,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_add(uint32_t* __restrict_
 
 }  // namespace
 
-bool scan_reserve(ScanScratch* s, size_t n, std::string* err) {
+bool scan_reserve(ScanScratch* s, size_t n, std::string* err, bool* full) {
   const size_t blocks = (n + kScanBlock - 1) / kScanBlock + 1;
   if (s->capacity >= n && s->block_sums) return true;
   scan_release(s);
@@ -83,6 +83,7 @@ bool scan_reserve(ScanScratch* s, size_t n, std::string* err) {
   if (e == hipSuccess) e = hipHostMalloc(&s->host_total, sizeof(uint32_t), hipHostMallocDefault);
   if (e != hipSuccess) {
     if (err) *err = std::string("scan: allocation failed: ") + hipGetErrorString(e);
+    if (full) *full = e == hipErrorOutOfMemory;
     scan_release(s);
     return false;
   }

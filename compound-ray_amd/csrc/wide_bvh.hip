@@ -300,7 +300,6 @@ struct Pool {
       if (err) *err = std::string("wide tree: hipMalloc: ") + hipGetErrorString(e);
       ok = false;
       full = e == hipErrorOutOfMemory;
-      if (full) (void)hipGetLastError();
       return nullptr;
     }
     held.push_back(p);
@@ -337,7 +336,7 @@ bool build(DeviceScene* S, Pool& pool, ScanScratch* scan, bool* unfit, hipStream
   int2* range = pool.get<int2>(2 * N - 1);
   int32_t* parent = pool.get<int32_t>(2 * N - 1);
   uint32_t* bad = pool.get<uint32_t>(1);
-  if (!pool.ok || !scan_reserve(scan, std::max((size_t)kRadix * tiles, N + 1), err)) return false;
+  if (!pool.ok || !scan_reserve(scan, std::max((size_t)kRadix * tiles, N + 1), err, &pool.full)) return false;
   float ext = 0.0f;
   for (int a = 0; a < 3; ++a) ext = std::max(ext, S->centroid_hi[a] - S->centroid_lo[a]);
   float radius = ext;
@@ -477,6 +476,7 @@ bool build_wide_tree(DeviceScene* scene, hipStream_t stream, std::string* err) {
   scan_release(&scan);
   if (ok || !pool.full) return ok;
   // no room: packets walk the 4-wide tree
+  (void)hipGetLastError();
   if (err) err->clear();
   return true;
 }
