@@ -49,8 +49,11 @@ std::vector<LaunchShape> LaunchTuner::candidates(int capacity) {
 }
 
 std::string LaunchTuner::key_of(const DeviceScene& scene, const UnitLaunch& U, uint64_t samples_per_pose) {
+  // The last word names the kernels that the shapes were timed on: files hold
+  // shapes of others too (traversal 1 was once another walk, and blocks a
+  // persistent grid's), which must not pass for these.
   char buf[160];
-  std::snprintf(buf, sizeof(buf), "tris%d_nodes%d_leaf%d_omm%d_spp%llu_stats%d_rec%d", scene.tri_count,
+  std::snprintf(buf, sizeof(buf), "tris%d_nodes%d_leaf%d_omm%d_spp%llu_stats%d_rec%d_wide64", scene.tri_count,
                 scene.node_count, scene.leaf_max, U.omm_count, (unsigned long long)samples_per_pose,
                 U.stats ? 1 : 0, U.samples ? 1 : 0);
   return buf;
