@@ -40,7 +40,8 @@ SceneView view_of(const DeviceScene& s) {
   v.textures = s.textures;
   float ext = 0.0f;
   for (int a = 0; a < 3; ++a) ext = std::max(ext, s.centroid_hi[a] - s.centroid_lo[a]);
-  v.wide = WideTree{s.wide_nodes, s.wide_tris, s.wide_root, s.wide_stack, ext * kPacketSpread, 4.0f * s.wide_radius};
+  v.wide = WideTree{s.wide_nodes, s.wide_tris, s.wide_root, s.wide_stack, ext * kPacketSpread,
+                    kWideRange * s.wide_radius};
   v.node_count = s.node_count;
   v.sky_mode = s.sky_mode;
   v.fault = s.fault;

@@ -43,7 +43,7 @@ constexpr int kWideLeaf = 4;     // triangles per leaf, at most
 // tree that could need more is walked through the 4-wide tree instead.
 constexpr int kWideStackMax = 512;
 
-// Relative padding of box tests: eight times the rounding of a test.
+// Relative padding of box tests.
 constexpr float kWidePad = 4.76837158203125e-7f;   // 2^-21
 
 // Scenes with a vertex that is not a number or further out than this have no
@@ -56,8 +56,16 @@ constexpr float kWideFarthest = 1.152921504606846976e18f;   // 2^60
 // Boxes as centre and half extent: (c - o) / d -/+ h / |d| needs no choice of
 // near and far planes.  Half extents are rounded up and padded by kWidePad of
 // themselves, of the centre and of the scene's radius R (the largest
-// coordinate): that covers the rounding of box tests for origins out to
-// 4 R, so no box loses a triangle that its ray hits.
+// coordinate).  With u = 2^-24, a test of an axis is off, as a length, by at most
+//   2 u (|c - o| + h)  the reciprocal, to one ulp
+//   u |o|              its product with the origin
+//   u |c - o|          the first FMA
+//   u (|c - o| + h)    the second
+// together 5 u |o| + 4 u |c| + 3 u h.  kWidePad = 8 u covers that for origins out
+// to kWideRange R, so that no box loses a ray that meets it.  (At 3.9 R, of 8 M
+// hits on corners of flat boxes one was lost.)  Packets from further out pad
+// the boxes by their own origins, walk64's kFar.
+constexpr float kWideRange = 1.5f;
 struct WideChild {
   float cx, cy, cz;
   int32_t ref;                 // bvh_format.h's encoding: a node, a leaf of the wide order, or kChildEmpty
