@@ -35,6 +35,7 @@ struct DeviceScene {
   int wide_root = 0;
   int wide_stack = 0;              // deferred children any packet can hold
   float wide_radius = 0.0f;        // the boxes' padding covers origins out to kWideRange of it
+  float wide_farthest = 0.0f;      // the largest coordinate of any vertex
   int tri_count = 0;
   int stack_bound = 0;             // deepest traversal stack any ray can need
   int levels = 0;

@@ -315,6 +315,7 @@ __device__ __forceinline__ void walk64(const WideNode64* nodes, const float4* wt
 constexpr float kPacketSlope = 1.0f;
 constexpr float kPacketSpread = 1.0f / 256.0f;
 constexpr float kFarStart = 1e30f;
+constexpr float kLeastComponent = 1e-37f;   // per unit of the scene's coordinates
 
 // The offsets and depths of B for rays that start `back` <= 0 times d behind
 // their origins o, all of them within `out` of 0 along each axis.  From starts
@@ -346,6 +347,7 @@ struct WideTree {
   int stack;      // LDS entries per wave
   float spread;   // how far apart the origins of one packet may be
   float range;    // origins this far out are covered by the boxes' padding
+  float least;    // smaller direction components count as this
 };
 
 __device__ __forceinline__ void closest_hit_wide(const WideTree& T, const Ray& ray, const RayPre& rp, bool active,
@@ -368,9 +370,13 @@ __device__ __forceinline__ void closest_hit_wide(const WideTree& T, const Ray& r
   r.okz = comp(rp.ox, rp.oy, rp.oz, rp.kz);
   r.sx = rp.sx; r.sy = rp.sy; r.sz = rp.sz;
   r.k = rp.kx | rp.ky << 2 | rp.kz << 4;
-  r.ix = __builtin_amdgcn_rcpf(fabsf(ray.dx) < 1e-30f ? copysignf(1e-30f, ray.dx) : ray.dx);
-  r.iy = __builtin_amdgcn_rcpf(fabsf(ray.dy) < 1e-30f ? copysignf(1e-30f, ray.dy) : ray.dy);
-  r.iz = __builtin_amdgcn_rcpf(fabsf(ray.dz) < 1e-30f ? copysignf(1e-30f, ray.dz) : ray.dz);
+  // A component near 0 counts as one whose reciprocal times any coordinate of the
+  // scene is finite; what that moves a point sideways is far below the boxes'
+  // padding.  (From an origin so far out that the product is not, the ray runs
+  // past every box, as its test then finds.)
+  r.ix = __builtin_amdgcn_rcpf(fabsf(ray.dx) < T.least ? copysignf(T.least, ray.dx) : ray.dx);
+  r.iy = __builtin_amdgcn_rcpf(fabsf(ray.dy) < T.least ? copysignf(T.least, ray.dy) : ray.dy);
+  r.iz = __builtin_amdgcn_rcpf(fabsf(ray.dz) < T.least ? copysignf(T.least, ray.dz) : ray.dz);
   r.nx = -(ray.ox * r.ix); r.ny = -(ray.oy * r.iy); r.nz = -(ray.oz * r.iz);
   // A ray with a not-a-number, a vanishing direction or an origin beyond
   // 1e30 hits nothing: its shears or distances are not numbers or exceed tmax.

@@ -41,7 +41,7 @@ SceneView view_of(const DeviceScene& s) {
   float ext = 0.0f;
   for (int a = 0; a < 3; ++a) ext = std::max(ext, s.centroid_hi[a] - s.centroid_lo[a]);
   v.wide = WideTree{s.wide_nodes, s.wide_tris, s.wide_root, s.wide_stack, ext * kPacketSpread,
-                    kWideRange * s.wide_radius};
+                    kWideRange * s.wide_radius, std::max(1e-30f, s.wide_farthest * kLeastComponent)};
   v.node_count = s.node_count;
   v.sky_mode = s.sky_mode;
   v.fault = s.fault;
@@ -561,7 +561,7 @@ __device__ __forceinline__ SceneView walk_view(KernelArgs* K) {
   S.nodes = K->S.nodes;
   S.tris = K->S.tris;
   S.wide = WideTree{K->S.wide.nodes, K->S.wide.tris, K->S.wide.root, K->S.wide.stack, K->S.wide.spread,
-                    K->S.wide.range};
+                    K->S.wide.range, K->S.wide.least};
   S.node_count = K->S.node_count;
   S.fault = K->S.fault;
   return S;

@@ -446,7 +446,9 @@ bool build(DeviceScene* S, Pool& pool, ScanScratch* scan, bool* unfit, hipStream
                      parents, total, made, n, bad);
   uint32_t wrong = 0;
   int32_t need = 0;
+  float box[6];
   if (!good(hipGetLastError(), "launch", err) ||
+      !good(hipMemcpyAsync(box, cur.box, sizeof(box), hipMemcpyDeviceToHost, stream), "box", err) ||
       !good(hipMemcpyAsync(&wrong, bad, sizeof(wrong), hipMemcpyDeviceToHost, stream), "check", err) ||
       !good(hipMemcpyAsync(&need, cur.need, sizeof(need), hipMemcpyDeviceToHost, stream), "bound", err) ||
       !good(hipStreamSynchronize(stream), "build", err))
@@ -461,6 +463,8 @@ bool build(DeviceScene* S, Pool& pool, ScanScratch* scan, bool* unfit, hipStream
   S->wide_root = total - 1;
   S->wide_stack = std::max(need, 1);
   S->wide_radius = radius;
+  S->wide_farthest = 0.0f;
+  for (float v : box) S->wide_farthest = std::max(S->wide_farthest, std::fabs(v));
   return true;
 }
 
