@@ -378,8 +378,9 @@ __device__ __forceinline__ void closest_hit_wide(const WideTree& T, const Ray& r
   r.iy = __builtin_amdgcn_rcpf(fabsf(ray.dy) < T.least ? copysignf(T.least, ray.dy) : ray.dy);
   r.iz = __builtin_amdgcn_rcpf(fabsf(ray.dz) < T.least ? copysignf(T.least, ray.dz) : ray.dz);
   r.nx = -(ray.ox * r.ix); r.ny = -(ray.oy * r.iy); r.nz = -(ray.oz * r.iz);
-  // A ray with a not-a-number, a vanishing direction or an origin beyond
-  // 1e30 hits nothing: its shears or distances are not numbers or exceed tmax.
+  // A ray with a not-a-number or an origin beyond 1e30 hits nothing: its shears
+  // or the triangle test's products are not numbers.  Directions beyond these
+  // lengths are the caller's to scale.
   const float size = fabsf(ray.dx) + fabsf(ray.dy) + fabsf(ray.dz);
   const float far = fmaxf(fmaxf(fabsf(ray.ox), fabsf(ray.oy)), fabsf(ray.oz));
   uint64_t left = __ballot(active && size > 1e-36f && size < 1e37f && far < 1e30f);

@@ -1190,21 +1190,36 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_rays(SceneView S, const
 // triangles 366 / 70 / 127, 5,000 511 / 172 / 228, 50,000 490 / 275 / 284,
 // 300,007 1,253 / 1,181 / 1,183; in 19,602 triangles 500 146 / 53 / 71, 50,000
 // 250 / 187 / 190, 300,007 728 / 844 / 808.
+//
+// Directions may have any length: beyond what the walk computes with (or where
+// the distances' products come near subnormal numbers) they are scaled by a
+// power of two, and the distances with them, exactly.
 constexpr float kRaySlope = 0.0625f;
+__device__ __forceinline__ int length_exponent(const Ray& ray) {
+  const float big = fmaxf(fmaxf(fabsf(ray.dx), fabsf(ray.dy)), fabsf(ray.dz));
+  return big < 0x1p-70f || big > 0x1p60f ? __builtin_amdgcn_frexp_expf(big) : 0;
+}
 __global__ __launch_bounds__(64, 6) void k_trace_packets(SceneView S, const Ray* __restrict__ rays, uint64_t n, int log,
                                                          int32_t* __restrict__ hit, float* __restrict__ tbb) {
   extern __shared__ uint32_t ray_lds[];
   const int lane = (int)(threadIdx.x & 63);
   const uint64_t r = ((uint64_t)blockIdx.x << log) + (uint64_t)lane;
   const bool inside = (lane >> log) == 0 && r < n;
-  const Ray ray = rays[inside ? r : 0];
+  Ray ray = rays[inside ? r : 0];
+  const int e = length_exponent(ray);
+  ray.dx = ldexpf(ray.dx, -e);
+  ray.dy = ldexpf(ray.dy, -e);
+  ray.dz = ldexpf(ray.dz, -e);
+  ray.tmin = ldexpf(ray.tmin, e);
+  ray.tmax = ldexpf(ray.tmax, e);
   Hit h;
   uint32_t steps = 0, tris = 0;
   closest_hit_wide(S.wide, ray, precompute_ray(ray), inside, reinterpret_cast<uint2*>(ray_lds), S.fault, h, steps,
                    tris, kRaySlope);
   if (!inside) return;
-  hit[r] = h.id == 0xffffffffu ? -1 : (int32_t)h.id;
-  tbb[3 * r] = h.t;
+  const bool miss = h.id == 0xffffffffu;
+  hit[r] = miss ? -1 : (int32_t)h.id;
+  tbb[3 * r] = miss ? rays[r].tmax : ldexpf(h.t, -e);
   tbb[3 * r + 1] = h.b1;
   tbb[3 * r + 2] = h.b2;
 }
