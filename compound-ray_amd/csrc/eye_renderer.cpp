@@ -586,6 +586,7 @@ double render_compound(EyeState& e, const Cam& c) {
     if (g_task_split == 2 && tasks_are_dealt(s.scene, U)) rec = plan = false;
     if (rec) {
       const uint32_t* before = e.d_split;
+      e.split_counts = nullptr;   // of the buffer that may go
       ensure_device(&e.d_split, &e.d_split_cap, (size_t)split_buffer_words(tasks));
       if (e.d_split != before) {   // new buffer: no steps recorded in it yet
         e.split_valid = false;
