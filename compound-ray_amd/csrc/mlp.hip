@@ -298,7 +298,7 @@ constexpr int kStage = stage_at(kStageLoss) + 1;    // floats per wave
 // without an index.  A wave takes tiles of 16 rows; a minibatch of the usual
 // size has one tile per wave, so the kernel is bound by a chain of latencies:
 // the weights into LDS, 72 dependent MFMAs per tile, the block's sums.  The
-// waves' sums meet in LDS, where the weights were (152 KB), and every
+// waves' sums meet in LDS, where the weights were (157 KB of 160), and every
 // parameter is added by one thread in wave order.  Written and added by one
 // wave after the other in global memory they took most of the kernel's time,
 // and a copy of the minibatch's rows a kernel before it: 4,096 rows 132 us
@@ -313,6 +313,7 @@ struct GradShared {
     float stage[kWaves][kStage];
   };
 };
+static_assert(sizeof(GradShared) <= 160 * 1024, "a workgroup's LDS");
 
 __global__ __launch_bounds__(kThreads) void k_grad(const float* __restrict__ x, const float* __restrict__ target,
                                                    const uint32_t* __restrict__ idx, int64_t n,

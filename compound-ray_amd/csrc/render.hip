@@ -508,7 +508,12 @@ __device__ __forceinline__ uint32_t xcd_run_block(uint32_t b, uint32_t blocks, u
 // through all slices before they exit).
 //
 // Packet variants: six waves per SIMD (at most 80 VGPRs); five and four are
-// 4 and 13 % slower on the bee eye's batch.  The per-ray variant's LDS stack
+// 4 and 13 % slower on the bee eye's batch.  The multi-pass instances spill at
+// six (68 bytes of scratch per lane, 84 with statistics; the uneven batch
+// writes 42 GB for 0.33 GB of colours), at five 8 and 16 bytes, at four none,
+// and are faster all the same: uneven batch 60.4 ms, 61.4 at five and 68.0 at
+// four; adaptive renders of the bee eye 13.0, 13.6 and 14.7, of 2.1 M
+// ommatidia 20.1, 20.6 and 22.0.  The per-ray variant's LDS stack
 // columns allow few resident blocks anyway; four waves (128 VGPRs) keep its
 // traversal loop free of scratch.
 //
@@ -1189,7 +1194,8 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_rays(SceneView S, const
 // traceRays, us, ray per lane / one ray per wave / 8: 500 rays in 2.2 M
 // triangles 366 / 70 / 127, 5,000 511 / 172 / 228, 50,000 490 / 275 / 284,
 // 300,007 1,253 / 1,181 / 1,183; in 19,602 triangles 500 146 / 53 / 71, 50,000
-// 250 / 187 / 190, 300,007 728 / 844 / 808.
+// 250 / 187 / 190, 300,007 728 / 844 / 808 (the one size where a ray per lane
+// was faster; in the pieces of 131,072 rays that a call now makes of it, 638).
 //
 // Directions may have any length: beyond what the walk computes with (or where
 // the distances' products come near subnormal numbers) they are scaled by a

@@ -151,6 +151,7 @@ size_t getCurrentEyeSamples(float* samples, size_t count);
 
 /* Closest hits of arbitrary rays (8 floats each as above) against the loaded
  * scene: primIds[i] = scene triangle index or -1, tbb[i*3..] = (t, b1, b2).
+ * Threads may call it at the same time (the calls take turns).
  * Returns 0 on success, -1 on error. */
 int traceRays(const float* rays, size_t count, int32_t* primIds, float* tbb);
 
